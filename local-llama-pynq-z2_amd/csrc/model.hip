@@ -97,6 +97,8 @@ struct llm_model {
     int pf_cap = 0, prefill_on = 1;
     float *pf_x = nullptr, *pf_y = nullptr, *pf_q = nullptr, *pf_s = nullptr;
     float *pf_ml = nullptr, *pf_acc = nullptr; // attention slice partials
+    float *pf_sc = nullptr;                    // strict attention: score rows, pf_sc_n floats
+    size_t pf_sc_n = 0;
     int8_t *pf_a = nullptr;
     int *pf_ids = nullptr;
     // h of the SwiGLU in the gate/up GEMM's epilogue (the down GEMM's input; pf_a is the gate/up input then),
@@ -879,6 +881,23 @@ int prefill_alloc(llm_model *m, int M) {
     return 0;
 }
 
+// the strict attention's score rows for chunks of M tokens up to position `end` (grown, never per chunk: a prompt's
+// last chunk has its largest end)
+int prefill_alloc_strict(llm_model *m, int M, int end) {
+    if (!m->strict || !prefill_strict_rows(m->hs)) return 0;
+    const size_t need = prefill_strict_scratch_floats(M, m->info.n_heads, m->info.n_kv_heads, end);
+    if (need <= m->pf_sc_n) return 0;
+    if (m->pf_sc) hipFree(m->pf_sc);
+    m->pf_sc = nullptr;
+    m->pf_sc_n = 0;
+    if (hipMalloc(&m->pf_sc, need * 4) != hipSuccess) {
+        fprintf(stderr, "llm_prefill: cannot allocate the score rows of %d tokens up to position %d\n", M, end);
+        return -1;
+    }
+    m->pf_sc_n = need;
+    return 0;
+}
+
 // positions p0 .. p0 + M - 1 (token ids in host memory) through every layer; the residual stream of the chunk
 // is left in pf_x and its K/V rows in the caches
 int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
@@ -914,7 +933,9 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
     pa.att_ml = m->pf_ml;
     pa.att_acc = m->pf_acc;
     pa.strict = m->strict;
+    pa.simds = 4 * hip_cu_count(m->device);
     pa.flash_bf = m->pf_flash_bf;
+    pa.att_sc = m->pf_sc;
     pa.xb = m->pf_y; // strict attention rows: the QKV GEMM output is consumed by then
     HIP_OR_FAIL("llm_prefill", launch_p_embed(pa, m->st));
     PgemmArgs g;
@@ -923,7 +944,7 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
     g.xs = m->pf_s;
     g.y = m->pf_y;
     g.M = M;
-    g.simds = 4 * hip_cu_count(m->device);
+    g.simds = pa.simds;
     g.qflavor = m->qflavor;
     g.strict = m->strict;
     g.hq = m->pf_h;
@@ -995,7 +1016,8 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
 // partials, and (finalize) its argmax into gen[pos0 + n - 1].  Afterwards the step state is position
 // pos0 + n - 1, as after those forward() calls.
 int prefill_all(llm_model *m, const int *ids, int n, bool sampled = false, int pos0 = 0) {
-    if (prefill_alloc(m, std::min(n, PREFILL_CHUNK))) return -1;
+    const int chunk = std::min(n, PREFILL_CHUNK);
+    if (prefill_alloc(m, chunk) || prefill_alloc_strict(m, chunk, pos0 + n)) return -1;
     for (int i = 0; i < n; i += PREFILL_CHUNK) {
         const int M = std::min(PREFILL_CHUNK, n - i);
         if (prefill_chunk(m, ids + i, pos0 + i, M)) return -1;
@@ -1019,7 +1041,7 @@ void free_model(llm_model *m) {
     if (m->hist) hipFree(m->hist);
     for (void *p : {(void *)m->pf_x, (void *)m->pf_y, (void *)m->pf_q, (void *)m->pf_s,
                     (void *)m->pf_a, (void *)m->pf_ids, (void *)m->pf_ml, (void *)m->pf_acc, (void *)m->pf_h,
-                    (void *)m->pf_hs})
+                    (void *)m->pf_hs, (void *)m->pf_sc})
         if (p) hipFree(p);
     if (m->st) hipStreamDestroy(m->st);
     if (m->file) munmap((void *)m->file, m->file_size);

@@ -86,10 +86,12 @@ struct ProwArgs {           // per-token elementwise kernels
     int n_heads, n_kv;
     int strict;             // 1: reference order (sequential RMSNorm sum, reference-order attention, libm expf)
     float *xb;              // strict attention: [M][dim] output rows before quantization
+    float *att_sc;          // strict attention: score rows, prefill_strict_scratch_floats()
     // attention slices: positions of token m in slices of att_sl, at most att_smax per token; partials
     // ml [M][n_heads][att_smax][2] (max, sum of exp) and acc [M][n_heads][att_smax][hs]
     int att_sl, att_smax;
     float *att_ml, *att_acc;
+    int simds;              // SIMDs of the device (0: 1024)
     int flash_bf;           // 1: the slice kernel's products on bf16 MFMA over split operands (head sizes % 32 == 0)
 };
 
@@ -102,6 +104,14 @@ static inline void prefill_att_slices(int end, int *sl, int *smax) {
     *smax = (end + s - 1) / s;
 }
 #define PREFILL_ATT_SMAX 16
+
+// The strict attention's row kernel takes these head sizes; its score rows hold SP floats (whole tiles of 64
+// positions up to `end`), n_kv x (M kv_mul rows rounded up to the 16 of a block).
+static inline bool prefill_strict_rows(int hs) { return hs == 16 || hs == 32 || hs == 48 || hs == 64 || hs == 128; }
+static inline int prefill_strict_sp(int end) { return (end + 63) / 64 * 64; }
+static inline size_t prefill_strict_scratch_floats(int M, int n_heads, int n_kv, int end) {
+    return (size_t)n_kv * (((size_t)M * (n_heads / n_kv) + 15) / 16 * 16) * prefill_strict_sp(end);
+}
 
 hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStream_t st);
 hipError_t launch_p_embed(const ProwArgs &a, hipStream_t st);

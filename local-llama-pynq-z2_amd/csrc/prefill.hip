@@ -7,6 +7,7 @@
 // group order, which is the reference's matmul (qwen.c:436-456, runq.c:429-458) for every (row, token).
 // The element-wise steps of forward() run per token, and attention is causal over the KV cache.
 #include <type_traits>
+#include <utility>
 
 #include "attn.h"
 #include "prefill.h"
@@ -1188,232 +1189,276 @@ __global__ void __launch_bounds__(256) k_p_attn_strict(ProwArgs a) {
                      a.p0 + m + 1, sm, a.xb + (size_t)m * a.dim + (size_t)h * hs);
 }
 
-// Strict prefill attention over tiles of tokens (qwen.c:526-546 for each token and head, in the reference's
-// order): block = (kv head, G consecutive tokens); its rows are the tokens x the kv head's query heads, so one
-// staging of a K or V tile (SPA_T positions, shared by every row) serves G x kv_mul heads.  Each (row,
-// position) score is the sequential dot q . k over the head's elements, then / sqrtf(hs), kept in LDS (rows of
-// SP floats, the launcher's bound on the positions); the row's maximum; expf(s - max) (ref_expf); the sum in
-// position order (one lane per row, all rows of the block in one wave: one wave64 add per position); the
-// division; then out[e] accumulated in position order over the V tiles, a (row, element) pair per thread.
-#define SPA_T 64 // positions per K/V tile
-#define SPA_NS 4 // score chains per thread and tile (rows x SPA_T <= 4 x 256)
-__host__ __device__ inline size_t spa_lds_floats(int rows, int hs, int sp) {
-    return (size_t)rows * hs + (size_t)rows * sp + (size_t)SPA_T * (hs + 4) + 2 * (size_t)rows;
+// Strict prefill attention (qwen.c:526-546 for each token and head, in the reference's order), a few rows per wave.
+//
+// A row is a (token, query head) pair; the rows of a kv head are its tokens in order x its kv_mul query heads, and a
+// wave owns R of them through all phases, with no exchange between waves but the shared K tiles.  Every running sum
+// is the reference's chain, and what is uniform over the wave in a chain's step is a DPP operand of the multiply
+// (row_newbcast: lane i of each row of 16 lanes), so a step costs its multiply and its add and nothing else:
+//   scores: lane = position.  The row's query is spread over registers (lane l of register c holds element
+//     16 c + l % 16), a K tile of SPW_T positions sits in LDS, shared by the block's waves; each score is the
+//     sequential dot over the head's elements, / sqrtf(hs), kept in the row's scratch in global memory (written and
+//     read back by the same lane);
+//   softmax: the row's maximum, expf (ref_expf) per position, and the sum in position order: the tile's exponentials
+//     go through a small LDS tile of the wave, lane r adds row r;
+//   values: lane = element (two per lane for a head size of 128).  The probabilities e / sum of a tile go through
+//     the same LDS tile into the DPP layout, V rows come straight from memory, 16 positions in flight ahead.
+// The floor is the 4 VALU instructions per row, position and 64 elements (multiply and add are rounded separately,
+// so there is no FMA and no MFMA in it).  Positions past a row's own token take no part (they are selected away, so
+// nothing that a later token holds can reach the row).
+//
+// More rows per wave share its loads and overheads, fewer give more waves (the launcher's rule).  Measured, per layer:
+// 512 tokens of the Qwen2-0.5B shape 51.6 us with a tile of rows per block and LDS-fed chains, now 40; 2011 tokens in
+// one launch 283-308 us for 184 us of multiplies and adds (39.3 T lane operations/s), 980 us before.
+#define SPW_T 64
+__host__ __device__ inline int spw_rows_pad(int M, int kv_mul) { return (M * kv_mul + 15) / 16 * 16; }
+template <int I>
+__device__ __forceinline__ float row_bcast(float x) { // lane I of each row of 16 lanes
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + I, 0xF, 0xF, true));
 }
-// One tile of G tokens (from m0) of kv head kvh; NV: value chains per thread (rows x hs <= NV x 256).
-template <int HS, int NV>
-__device__ __forceinline__ void spa_tile(const ProwArgs &a, int G, int SP, int kvh, int m0, float *sm) {
-    const int hs = HS ? HS : a.head_size, kv_mul = a.n_heads / a.n_kv;
-    const int gn = min(G, a.M - m0), R = gn * kv_mul, Rmax = G * kv_mul;
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE, HP = hs + 4, hs4 = hs / 4;
-    const int Pmax = a.p0 + m0 + gn; // positions of the tile's last token
-    float *qs = sm, *sc = qs + (size_t)Rmax * hs, *kv = sc + (size_t)Rmax * SP, *rmax = kv + SPA_T * HP,
-          *rsum = rmax + Rmax;
-    const int koff = kvh * hs;
-    auto row_pos = [&](int r) { return a.p0 + m0 + r / kv_mul + 1; };          // P of row r
-    auto row_head = [&](int r) { return kvh * kv_mul + r % kv_mul; };          // query head of row r
-    auto row_tok = [&](int r) { return m0 + r / kv_mul; };                     // token of row r
-    __syncthreads(); // a previous tile's rows are consumed
-    for (int r = wave; r < R; r += 4)
-        for (int c = lane; c < hs4; c += WAVE)
-            ((float4 *)(qs + r * hs))[c] = *(const float4 *)(a.q + (size_t)row_tok(r) * a.dim + (size_t)row_head(r) * hs + 4 * c);
-    // a K or V tile: positions t0 .. t0 + SPA_T - 1 (below Pmax) of the kv head, rows of hs + 4 floats in LDS;
-    // fetch() puts all of a thread's loads (SPA_T x hs / 1024 vectors) in flight at once, put() stores them
-    constexpr int FV = (HS ? HS : 256) * SPA_T / 1024; // vectors per thread (hs <= 256)
-    // (buffer loads: a position past the range reads zeros through an out-of-range offset, so every load is issued
-    // unconditionally and each staging waits for its own tile's loads only)
-    const int nrec = (int)(((size_t)(Pmax - 1) * a.kv_dim + hs) * 4);
-    const auto rs_k = __builtin_amdgcn_make_buffer_rsrc((void *)(a.kc + koff), 0, nrec, 0x00020000);
-    const auto rs_v = __builtin_amdgcn_make_buffer_rsrc((void *)(a.vc + koff), 0, nrec, 0x00020000);
-    auto fetch = [&](__amdgpu_buffer_rsrc_t rs, int t0, float4 (&f)[FV]) {
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
+
+// acc[k] = acc[k] + b_k * x[i][k % VE] for i = 0 .. 15 in order, b_k lane i (of each 16) of w[k / VE]: the products of
+// a few steps first, then their adds, so that no product's register is written again within the two instructions
+// that a DPP operand has to wait for (the compiler fills them with no-ops otherwise).  keep(i, k) false leaves acc[k].
+template <int N, int VE, typename K>
+__device__ __forceinline__ void chain16(float (&acc)[N], const float (&w)[N / VE], const float (&x)[16][VE], K &&keep) {
+    constexpr int G = N >= 4 ? 1 : 4 / N; // steps a batch
+    static_for<16 / G>([&](auto b) {
+        float p[G][N];
+        static_for<G>([&](auto g) {
+            constexpr int i = b.value * G + g.value;
 #pragma unroll
-        for (int j = 0; j < FV; j++) {
-            const int idx = tid + 256 * j, tt = idx / hs4, c = idx - tt * hs4;
-            const bool ok = tt < SPA_T && t0 + tt < Pmax;
-            const auto v = __builtin_amdgcn_raw_buffer_load_b128(
-                rs, ok ? (uint32_t)((t0 + tt) * a.kv_dim + 4 * c) * 4u : 0x80000000u, 0, 0);
-            f[j] = *(const float4 *)&v;
-        }
-    };
-    auto put = [&](const float4 (&f)[FV]) {
+            for (int k = 0; k < N; k++) p[g.value][k] = row_bcast<i>(w[k / VE]) * x[i][k % VE];
+        });
+        __builtin_amdgcn_sched_barrier(0x3f4); // (only vector arithmetic keeps its side of this)
 #pragma unroll
-        for (int j = 0; j < FV; j++) {
-            const int idx = tid + 256 * j, tt = idx / hs4, c = idx - tt * hs4;
-            if (HS || tt < SPA_T) *(float4 *)(kv + tt * HP + 4 * c) = f[j]; // (a fixed head size fills FV exactly)
-        }
-    };
-    // DK tiles in flight: a tile's compute is shorter than a round trip to the cache, so the loads of the tiles
-    // DK ahead leave as each tile is staged (register sets used in turn, the tile loop unrolled by DK)
-    constexpr int DK = (HS && HS <= 64) ? 4 : 2;
-    float4 fr[DK][FV];
-    const int nkt = (Pmax + SPA_T - 1) / SPA_T;
-    KERNEL_MARK(0);
-    const float rs = sqrtf((float)hs);
-    // (1) scores: thread tid takes position tt = tid % 64 of the tile for rows tid / 64 + 4 j (j < SPA_NS), its
-    // K row read once per 4 elements for all of them; each score the sequential dot over the head's elements
-    const int s_tt = tid % SPA_T, s_r0 = tid / SPA_T;
+        for (int g = 0; g < G; g++)
 #pragma unroll
-    for (int dd = 0; dd < DK; dd++) fetch(rs_k, dd * SPA_T, fr[dd]); // (tiles past the range: zeros, no traffic)
-    for (int k0 = 0; k0 < nkt; k0 += DK)
-#pragma unroll
-    for (int dd = 0; dd < DK; dd++) {
-        const int kt = k0 + dd, t0 = kt * SPA_T;
-        if (kt >= nkt) break;
-        __syncthreads(); // the previous tile is consumed
-        put(fr[dd]);
-        __syncthreads();
-        fetch(rs_k, (kt + DK) * SPA_T, fr[dd]);
-        float d[SPA_NS];
-#pragma unroll
-        for (int j = 0; j < SPA_NS; j++) d[j] = 0.0f;
-        const float4 *kr = (const float4 *)(kv + s_tt * HP);
-        const float4 *qr[SPA_NS];
-#pragma unroll
-        for (int j = 0; j < SPA_NS; j++) qr[j] = (const float4 *)(qs + min(s_r0 + 4 * j, Rmax - 1) * hs);
-#pragma unroll 4
-        for (int c = 0; c < hs4; c++) {
-            const float4 k4 = kr[c];
-#pragma unroll
-            for (int j = 0; j < SPA_NS; j++) {
-                const float4 q4 = qr[j][c];
-                d[j] += q4.x * k4.x;
-                d[j] += q4.y * k4.y;
-                d[j] += q4.z * k4.z;
-                d[j] += q4.w * k4.w;
+            for (int k = 0; k < N; k++) {
+                const float s = acc[k] + p[g][k];
+                acc[k] = keep(b.value * G + g, k) ? s : acc[k];
             }
-        }
-        const int t = t0 + s_tt;
-#pragma unroll
-        for (int j = 0; j < SPA_NS; j++) {
-            const int r = s_r0 + 4 * j;
-            if (r < R && t < row_pos(r)) sc[(size_t)r * SP + t] = d[j] / rs;
-        }
-    }
-    __syncthreads();
-    KERNEL_MARK(1);
-    // (2) a wave per row: its maximum, then its exponentials (positions past the row, up to the tile's last
-    // token's, set to 0: the sums below then add +0 there, which leaves a positive sum unchanged)
-    for (int r = wave; r < R; r += 4) {
-        float *row = sc + (size_t)r * SP;
-        const int P = row_pos(r);
-        float mx = -INFINITY;
-        for (int t = lane; t < P; t += WAVE) mx = fmaxf(mx, row[t]);
-        mx = wave_max(mx);
-        for (int t = lane; t < Pmax; t += WAVE) row[t] = t < P ? ref_expf(row[t] - mx) : 0.0f;
-    }
-    __syncthreads();
-    KERNEL_MARK(2);
-    // (3) the sums in position order: lane r of wave 0 adds row r, 8 positions in flight
-    if (wave == 0 && lane < R) {
-        const float *row = sc + (size_t)lane * SP;
-        const float4 *row4 = (const float4 *)row;
-        float s = 0.0f;
-        int t = 0;
-        for (; t + 8 <= Pmax; t += 8) {
-            const float4 v0 = row4[t / 4], v1 = row4[t / 4 + 1];
-            s = s + v0.x;
-            s = s + v0.y;
-            s = s + v0.z;
-            s = s + v0.w;
-            s = s + v1.x;
-            s = s + v1.y;
-            s = s + v1.z;
-            s = s + v1.w;
-        }
-        for (; t < Pmax; t++) s = s + row[t];
-        rsum[lane] = s;
-    }
-    __syncthreads();
-    KERNEL_MARK(3);
-    // the probabilities (0 stays 0 past the row: the value sums add +0 there)
-    for (int r = wave; r < R; r += 4) {
-        float *row = sc + (size_t)r * SP;
-        const float sum = rsum[r];
-        for (int t = lane; t < Pmax; t += WAVE) row[t] = row[t] / sum;
-    }
-    KERNEL_MARK(4);
-    // (4) values: thread tid takes element e = tid % hs of rows tid / hs + (256 / hs) j, the V element read once
-    // per position for all of them; positions in order over the tiles
-    const int v_e = tid % hs, v_r0 = tid / hs, v_rs = 256 / hs;
-    float acc[NV];
-    const float *pr[NV];
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        acc[j] = 0.0f;
-        pr[j] = sc + (size_t)min(v_r0 + v_rs * j, Rmax - 1) * SP;
-    }
-#pragma unroll
-    for (int dd = 0; dd < DK; dd++) fetch(rs_v, dd * SPA_T, fr[dd]);
-    for (int k0 = 0; k0 < nkt; k0 += DK)
-#pragma unroll
-    for (int dd = 0; dd < DK; dd++) {
-        const int kt = k0 + dd, t0 = kt * SPA_T;
-        if (kt >= nkt) break;
-        __syncthreads(); // the probabilities are written, the previous tile consumed
-        put(fr[dd]);
-        __syncthreads();
-        fetch(rs_v, (kt + DK) * SPA_T, fr[dd]);
-        const int T = min(SPA_T, Pmax - t0);
-        const float *vt = kv + v_e;
-        int tt = 0;
-        // 4 positions a step: each row's 4 weights in one load (rows and t0 are 16-byte aligned), then the
-        // products and adds position by position; a full tile as straight-line code (the loads of later steps
-        // scheduled ahead of earlier steps' arithmetic)
-        auto step4 = [&](int s) {
-            const float v0 = vt[s * HP], v1 = vt[(s + 1) * HP], v2 = vt[(s + 2) * HP], v3 = vt[(s + 3) * HP];
-#pragma unroll
-            for (int j = 0; j < NV; j++) {
-                const float4 w = *(const float4 *)(pr[j] + t0 + s);
-                acc[j] += w.x * v0;
-                acc[j] += w.y * v1;
-                acc[j] += w.z * v2;
-                acc[j] += w.w * v3;
-            }
-        };
-        if (T == SPA_T) {
-#pragma unroll
-            for (int s = 0; s < SPA_T; s += 4) step4(s);
-            tt = SPA_T;
-        }
-        for (; tt + 4 <= T; tt += 4) {
-            const float v0 = vt[tt * HP], v1 = vt[(tt + 1) * HP], v2 = vt[(tt + 2) * HP], v3 = vt[(tt + 3) * HP];
-#pragma unroll
-            for (int j = 0; j < NV; j++) {
-                const float4 w = *(const float4 *)(pr[j] + t0 + tt);
-                acc[j] += w.x * v0;
-                acc[j] += w.y * v1;
-                acc[j] += w.z * v2;
-                acc[j] += w.w * v3;
-            }
-        }
-        for (; tt < T; tt++) {
-            const float v = vt[tt * HP];
-#pragma unroll
-            for (int j = 0; j < NV; j++) acc[j] += pr[j][t0 + tt] * v;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        const int r = v_r0 + v_rs * j;
-        if (r < R) a.xb[(size_t)row_tok(r) * a.dim + (size_t)row_head(r) * hs + v_e] = acc[j];
-    }
-    KERNEL_MARK(5);
+        __builtin_amdgcn_sched_barrier(0x3f4);
+    });
 }
 
-// Strict prefill attention over tiles of tokens (qwen.c:526-546 for each token and head, in the reference's
-// order): a tile = G consecutive tokens of one kv head; its rows are the tokens x the kv head's query heads, so
-// one staging of a K or V tile (SPA_T positions, shared by every row) serves G x kv_mul heads.  Each (row,
-// position) score is the sequential dot q . k over the head's elements, then / sqrtf(hs), kept in LDS (rows of
-// SP floats, the launcher's bound on the positions); the row's maximum; expf(s - max) (ref_expf); the sum in
-// position order (one lane per row, every row of the tile in one wave: one wave64 add per position); the
-// division; then out[e] accumulated in position order over the V tiles, (row, element) chains per thread.
-// One tile per block, the longest causal ranges first (two blocks per CU at 512 tokens; pairing a short and a
-// long range in one block, every block the same work, measured 6% slower: fewer waves in flight per CU).
-template <int HS, int NV>
-__global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int G, int SP) {
-    extern __shared__ __align__(16) float sm[];
-    const int ntiles = (a.M + G - 1) / G, y = ntiles - 1 - (int)blockIdx.y;
-    spa_tile<HS, NV>(a, G, SP, blockIdx.x, y * G, sm);
+template <int HS, int R>
+__global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) {
+    constexpr int KP = HS + 4, NQ = HS / 16, VE = HS > 64 ? 2 : 1, FV = HS * SPW_T / 1024;
+    static_assert(HS % 16 == 0 && (HS <= 64 || HS == 128), "head sizes of the row kernel");
+    __shared__ __align__(16) float kt[SPW_T * KP];
+    __shared__ __align__(16) float et[4][R][SPW_T + 4];
+    const int tid = threadIdx.x, l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = l & 15;
+    const int kvh = blockIdx.x, kv_mul = a.n_heads / a.n_kv, rows = a.M * kv_mul;
+    // the longest causal ranges first
+    const int b0 = 4 * R * ((int)gridDim.y - 1 - (int)blockIdx.y), row0 = b0 + w * R;
+    int tok[R], head[R], P[R]; // (rows past the last one repeat it; their outputs are not stored)
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int rho = min(row0 + r, rows - 1);
+        tok[r] = rho / kv_mul;
+        head[r] = kvh * kv_mul + rho - tok[r] * kv_mul;
+        P[r] = a.p0 + tok[r] + 1;
+    }
+    const int Pw = P[R - 1], Pb = a.p0 + min(b0 + 4 * R - 1, rows - 1) / kv_mul + 1; // the wave's, the block's last
+    const int koff = kvh * HS, nrec = (int)(((size_t)(Pb - 1) * a.kv_dim + HS) * 4);
+    // (a position past the block's last reads zeros through an out-of-range offset)
+    const auto rs_k = __builtin_amdgcn_make_buffer_rsrc((void *)(a.kc + koff), 0, nrec, PG_RSRC3);
+    const auto rs_v = __builtin_amdgcn_make_buffer_rsrc((void *)(a.vc + koff), 0, nrec, PG_RSRC3);
+    float *scr[R];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        scr[r] = a.att_sc + ((size_t)kvh * spw_rows_pad(a.M, kv_mul) + row0 + r) * SP + l;
+
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    float mx[R];
+    {
+        float qv[R][NQ];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int c = 0; c < NQ; c++) qv[r][c] = a.q[(size_t)tok[r] * a.dim + head[r] * HS + 16 * c + l16];
+        float4 f[FV];
+        auto fetch = [&](int t0) {
+#pragma unroll
+            for (int j = 0; j < FV; j++) {
+                const int idx = tid + 256 * j, tt = idx / (HS / 4), c = idx - tt * (HS / 4);
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+                    rs_k, t0 + tt < Pb ? (uint32_t)((t0 + tt) * a.kv_dim + 4 * c) * 4u : 0x80000000u, 0, 0);
+                f[j] = *(const float4 *)&v;
+            }
+        };
+        const float rs = sqrtf((float)HS);
+#pragma unroll
+        for (int r = 0; r < R; r++) mx[r] = -INFINITY;
+        fetch(0);
+        for (int t0 = 0; t0 < Pb; t0 += SPW_T) {
+            __syncthreads(); // the previous tile is consumed
+#pragma unroll
+            for (int j = 0; j < FV; j++) {
+                const int idx = tid + 256 * j, tt = idx / (HS / 4), c = idx - tt * (HS / 4);
+                *(float4 *)(kt + tt * KP + 4 * c) = f[j];
+            }
+            __syncthreads();
+            fetch(t0 + SPW_T);
+            const float *kr = kt + l * KP;
+            float d[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) d[r] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NQ; c++) {
+                float kk[16][1], qc[R];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float4 k4 = *(const float4 *)(kr + 16 * c + 4 * j);
+                    kk[4 * j][0] = k4.x;
+                    kk[4 * j + 1][0] = k4.y;
+                    kk[4 * j + 2][0] = k4.z;
+                    kk[4 * j + 3][0] = k4.w;
+                }
+#pragma unroll
+                for (int r = 0; r < R; r++) qc[r] = qv[r][c];
+                chain16<R, 1>(d, qc, kk, [](int, int) { return true; });
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float s = d[r] / rs;
+                scr[r][t0] = s;
+                mx[r] = t0 + l < P[r] ? fmaxf(mx[r], s) : mx[r];
+            }
+        }
+    }
+    if (row0 >= rows) return; // the whole wave (no barrier below)
+
+    float sum[R];
+    {
+        float s = 0.0f; // lane l: the running sum of row l % R
+#pragma unroll
+        for (int r = 0; r < R; r++) mx[r] = wave_max(mx[r]);
+        float nx[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) nx[r] = scr[r][0];
+        for (int t0 = 0; t0 < Pw; t0 += SPW_T) {
+            float e[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) e[r] = nx[r];
+            const int tn = t0 + SPW_T < Pw ? t0 + SPW_T : t0;
+#pragma unroll
+            for (int r = 0; r < R; r++) nx[r] = scr[r][tn];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                e[r] = t0 + l < P[r] ? ref_expf(e[r] - mx[r]) : 0.0f; // (+0 leaves the sum, never -0, unchanged)
+                scr[r][t0] = e[r];
+                et[w][r][l] = e[r];
+            }
+            wave_sync();
+            const float4 *er = (const float4 *)et[w][l & (R - 1)];
+            float4 x[SPW_T / 4];
+#pragma unroll
+            for (int j = 0; j < SPW_T / 4; j++) x[j] = er[j];
+#pragma unroll
+            for (int j = 0; j < SPW_T / 4; j++) {
+                s = s + x[j].x;
+                s = s + x[j].y;
+                s = s + x[j].z;
+                s = s + x[j].w;
+            }
+            wave_sync();
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) sum[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), r));
+    }
+
+    float acc[R * VE];
+#pragma unroll
+    for (int k = 0; k < R * VE; k++) acc[k] = 0.0f;
+    {
+        const uint32_t vo = (HS >= 64 || l < HS ? l : 0) * 4 * VE;
+        const int vstep = a.kv_dim * 4;
+        float v[2][16][VE];
+        auto vload = [&](int k, int t0) { // V of positions t0 .. t0 + 15
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int so = min(t0 + i, Pb - 1) * vstep; // (past the last position: its row, selected away)
+                if constexpr (VE == 1) {
+                    v[k][i][0] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_v, vo, so, 0));
+                } else {
+                    const auto x = __builtin_amdgcn_raw_buffer_load_b64(rs_v, vo, so, 0);
+                    v[k][i][0] = __int_as_float(x[0]);
+                    v[k][i][1] = __int_as_float(x[1]);
+                }
+            }
+        };
+        float nx[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) nx[r] = scr[r][0];
+        vload(0, 0);
+        const int Pmin = P[0];
+        for (int t0 = 0; t0 < Pw; t0 += SPW_T) {
+#pragma unroll
+            for (int r = 0; r < R; r++) et[w][r][l] = nx[r] / sum[r];
+            wave_sync();
+            const int tn = t0 + SPW_T < Pw ? t0 + SPW_T : t0;
+#pragma unroll
+            for (int r = 0; r < R; r++) nx[r] = scr[r][tn];
+            float pr[R][4];
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) pr[r][c] = et[w][r][16 * c + l16];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int tc = t0 + 16 * c;
+                vload((c + 1) & 1, tc + 16);
+                float pc[R];
+#pragma unroll
+                for (int r = 0; r < R; r++) pc[r] = pr[r][c];
+                if (tc + 16 <= Pmin) chain16<R * VE, VE>(acc, pc, v[c & 1], [](int, int) { return true; });
+                else // positions that some row of the wave does not see
+                    chain16<R * VE, VE>(acc, pc, v[c & 1], [&](int i, int k) { return tc + i < P[k / VE]; });
+            }
+            wave_sync();
+        }
+    }
+    if (HS % a.gs) { // quantization groups that cross heads: k_p_quant_rows quantizes the rows afterwards
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if (row0 + r < rows && VE * l < HS) {
+                float *o = a.xb + (size_t)tok[r] * a.dim + head[r] * HS + VE * l;
+#pragma unroll
+                for (int e = 0; e < VE; e++) o[e] = acc[VE * r + e];
+            }
+        return;
+    }
+    // int8 quantization into the o projection's input (qwen.c:549, runq.c:571): a group is gs / VE lanes
+    const int MB = pf_blocks(a.M), gl = a.gs / VE; // 16, 32 or 64 lanes
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        float gm = 0.0f;
+#pragma unroll
+        for (int e = 0; e < VE; e++) gm = fmaxf(gm, fabsf(acc[VE * r + e]));
+        gm = max16(gm);
+        if (gl >= 32) gm = fmaxf(gm, __shfl_xor(gm, 16));
+        if (gl >= 64) gm = fmaxf(gm, __shfl_xor(gm, 32));
+        const float scale = quant_scale(gm, a.qflavor), inv = quant_inv(scale);
+        if (row0 + r < rows && VE * l < HS) {
+            const int k0 = head[r] * HS + VE * l;
+            int8_t *o = a.oq + pf_act_off(tok[r], k0, MB);
+#pragma unroll
+            for (int e = 0; e < VE; e++) o[e] = quant_one(acc[VE * r + e], scale, inv, a.qflavor);
+            if ((l & (gl - 1)) == 0) a.os[pf_scale_off(tok[r], k0 / a.gs, MB)] = scale;
+        }
+    }
 }
 
 // int8 quantization of the rows xb[m] (qwen.c:549, runq.c:571) into the o projection's input
@@ -1461,37 +1506,29 @@ hipError_t launch_p_attention(const ProwArgs &a, hipStream_t st) {
             ((uintptr_t)a.oq & 3) || lds > 65536 || a.n_heads % a.n_kv ||
             (size_t)(a.p0 + a.M + 64) * a.kv_dim * 4 >= 0x7fffffffu)
             return hipErrorInvalidValue;
-        // tiles of G tokens when their rows' scores fit LDS (G x kv_mul rows, positions up to p0 + M), else a
-        // block per (head, token) that streams the positions
-        // score rows of SP = 4 x odd floats: 16-byte aligned (the value chains read 4 weights a load) and the sums'
-        // lanes, one per row, on distinct banks
-        const int kvm = a.n_heads / a.n_kv, SP = 4 * (((a.p0 + a.M + 3) / 4) | 1);
-        int G = 0;
-        for (int g = 4; g >= 1 && !G; g /= 2)
-            if (g * kvm <= 4 * SPA_NS && g * kvm * hs <= 8 * 256 && hs <= 256 && 256 % hs == 0 &&
-                spa_lds_floats(g * kvm, hs, SP) * 4 <= 65536)
-                G = g;
-        if (G) {
-            const int ntiles = (a.M + G - 1) / G;
-            const dim3 grid(a.n_kv, ntiles);
-            const size_t sl = spa_lds_floats(G * kvm, hs, SP) * 4;
-            const bool nv4 = G * kvm * hs <= 4 * 256;
-#define SPA_LAUNCH(H)                                                                                          \
-            if (nv4) hipLaunchKernelGGL((k_p_attn_strict_rows<H, 4>), grid, dim3(256), sl, st, a, G, SP);      \
-            else hipLaunchKernelGGL((k_p_attn_strict_rows<H, 8>), grid, dim3(256), sl, st, a, G, SP);
-            if (hs == 64) {
-                SPA_LAUNCH(64)
-            } else if (hs == 128) {
-                SPA_LAUNCH(128)
-            } else {
-                SPA_LAUNCH(0)
+        if (prefill_strict_rows(hs)) {
+            const int kvm = a.n_heads / a.n_kv, rows = a.M * kvm, SP = prefill_strict_sp(a.p0 + a.M);
+            if (!a.att_sc) return hipErrorInvalidValue;
+            // rows per wave: 4 from 9 rows per SIMD, 2 from 3.5, else 1 (whole strict prefills of two layers, 1024 SIMDs,
+            // R = 4 / 2 / 1, us: Qwen2-0.5B shape 200 tokens, 2800 rows: 248 / 234 / 231; 300: 281 / 261 / 269; 512:
+            // 317 / 309 / 331; 1024, 14336 rows: 503 / 524 / 628; 7B shape 300, 8400 rows: 1034 / 1034 / 1072; 512:
+            // 1453 / 1473 / 1586)
+            const long all = (long)rows * a.n_kv, simds = a.simds > 0 ? a.simds : 1024;
+            const int R = all >= 9 * simds ? 4 : 2 * all >= 7 * simds ? 2 : 1;
+            const dim3 grid(a.n_kv, (rows + 4 * R - 1) / (4 * R));
+#define SPW_LAUNCH(H)                                                                                          \
+            if (hs == H) {                                                                                     \
+                if (R == 4) hipLaunchKernelGGL((k_p_attn_strict_rows<H, 4>), grid, dim3(256), 0, st, a, SP);   \
+                else if (R == 2) hipLaunchKernelGGL((k_p_attn_strict_rows<H, 2>), grid, dim3(256), 0, st, a, SP); \
+                else hipLaunchKernelGGL((k_p_attn_strict_rows<H, 1>), grid, dim3(256), 0, st, a, SP);          \
             }
-#undef SPA_LAUNCH
-        } else if (hs == 64) hipLaunchKernelGGL(k_p_attn_strict<64>, dim3(a.n_heads, a.M), dim3(256), lds, st, a);
-        else if (hs == 128) hipLaunchKernelGGL(k_p_attn_strict<128>, dim3(a.n_heads, a.M), dim3(256), lds, st, a);
-        else hipLaunchKernelGGL(k_p_attn_strict<0>, dim3(a.n_heads, a.M), dim3(256), lds, st, a);
+            SPW_LAUNCH(16) SPW_LAUNCH(32) SPW_LAUNCH(48) SPW_LAUNCH(64) SPW_LAUNCH(128)
+#undef SPW_LAUNCH
+        } else {
+            hipLaunchKernelGGL(k_p_attn_strict<0>, dim3(a.n_heads, a.M), dim3(256), lds, st, a);
+        }
         hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess || (prefill_strict_rows(hs) && hs % a.gs == 0)) return e;
         hipLaunchKernelGGL(k_p_quant_rows, dim3(a.M), dim3(256), (size_t)a.dim * 4, st, a);
         return hipGetLastError();
     }
