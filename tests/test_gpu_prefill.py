@@ -268,7 +268,7 @@ def test_prefill_split_bf16_attention_against_the_fp32_products(monkeypatch, tmp
 
 
 @pytest.mark.parametrize("fmt,shape,n,more", [("qwb", ("dim=896", "heads=14", "kv_heads=2"), 333, 1),
-                                              ("qwb", ("dim=896", "heads=14", "kv_heads=2"), 530, 70),
+                                              ("qwb", ("dim=256", "heads=4", "kv_heads=2"), 2100, 40),
                                               ("qwb", ("dim=512", "heads=4", "kv_heads=2"), 140, 21),
                                               ("qwb", ("dim=512", "heads=4", "kv_heads=1"), 2, 65),
                                               ("qwb", ("dim=384", "heads=8", "kv_heads=8"), 129, 3),
@@ -281,11 +281,12 @@ def test_strict_prefill_attention_equals_the_per_position_path(tmp_path, fmt, sh
     few rows), against as many decode steps, whose attention is another kernel: every layer's K/V rows (layers
     1 and 2 follow from the attention of all positions before them) and the last position's logits bit for bit.
     Head sizes 64 (7 query heads per kv head), 128, 48, 32, 16 and 96 (the general kernel), row counts below, at
-    and above a block's and a tile's 64 positions, two chunks of 512; the oracle's logits at the last position"""
+    and above a block's and a tile's 64 positions, two chunks of 2048; the oracle's logits at the last position"""
     end = n + more
-    extra = ["hidden=256", "layers=3", "vocab=512", "max_seq=700"] + (["head_k=256"] if fmt == "qwb" else [])
+    ctx = max(700, end)
+    extra = ["hidden=256", "layers=3", "vocab=512", f"max_seq={ctx}"] + (["head_k=256"] if fmt == "qwb" else [])
     p = synth(fmt, str(tmp_path / f"s.{fmt}"), "tiny", 7, *shape, *extra)
-    a, b = pkg().Model(p, 700), pkg().Model(p, 700)
+    a, b = pkg().Model(p, ctx), pkg().Model(p, ctx)
     hid = a.head_ids if fmt == "qwb" else np.arange(512)
     ids = [int(hid[v]) for v in np.random.default_rng(n).integers(0, len(hid), end)]
     for m in (a, b):
@@ -299,7 +300,7 @@ def test_strict_prefill_attention_equals_the_per_position_path(tmp_path, fmt, sh
     assert np.array_equal(a.forward(ids[-1], end - 1), lg)
     a.close()
     b.close()
-    om = OracleModel(p, 700)
+    om = OracleModel(p, ctx)
     for pos, t in enumerate(ids):
         ref = om.forward(t, pos)
     assert np.array_equal(lg, ref)
