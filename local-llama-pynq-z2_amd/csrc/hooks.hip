@@ -91,12 +91,14 @@ extern "C" int mvh_group_dots(const uint8_t *w, const int8_t *xq, int n, int d, 
 
 extern "C" int mvh_prefill_gemm(const uint8_t *w, const void *ws, const int8_t *xq, const float *xs, int M, int n,
                                 int d, int bits, int gs, int rb, int shape, float *y) {
+    const int fast = shape == 33; // k_pgemm32 with the fast mode's sums
+    if (fast) shape = PGEMM_SHAPE_32;
     const int wbits = bits == 0 ? 8 : bits, sf32 = bits == 0;
     if (!w || !ws || !xq || !xs || !y || M < 1 || n <= 0 || d <= 0 || d % 4 || n % 16 ||
         (bits != 0 && bits != 4 && bits != 8) || (gs != 32 && gs != 64) || (bits != 0 && gs != 32) || n % gs ||
-        (rb != 8 && rb != 16 && rb != 64) ||
+        (rb != 8 && rb != 16 && rb != 32 && rb != 64) ||
         (shape != 0 && shape != 11 && shape != 12 && shape != 14 && shape != 21 && shape != 22 && shape != 24 &&
-         shape != 41 && shape != 42)) {
+         shape != 41 && shape != 42 && shape != PGEMM_SHAPE_32)) {
         fprintf(stderr, "mvh_prefill_gemm: bad arguments (M=%d n=%d d=%d bits=%d gs=%d rb=%d shape=%d)\n", M, n, d,
                 bits, gs, rb, shape);
         return -1;
@@ -117,7 +119,7 @@ extern "C" int mvh_prefill_gemm(const uint8_t *w, const void *ws, const int8_t *
     std::vector<int8_t> xt(abytes, 0);
     std::vector<float> st(sfl, 0.0f);
     for (int m = 0; m < M; m++) {
-        for (int k = 0; k < n; k++) xt[pf_act_off(m, k, MB)] = xq[(size_t)m * n + k];
+        for (int k = 0; k < n; k++) xt[pf_act(m, k, M, shape == PGEMM_SHAPE_32)] = xq[(size_t)m * n + k];
         for (int g = 0; g < ng; g++) st[pf_scale_off(m, g, MB)] = xs[(size_t)m * ng + g];
     }
     int rc = -1;
@@ -145,6 +147,7 @@ extern "C" int mvh_prefill_gemm(const uint8_t *w, const void *ws, const int8_t *
         g.y = dy;
         g.M = M;
         g.shape = shape;
+        g.strict = !fast;
         int dev = 0;
         hipGetDevice(&dev);
         g.simds = 4 * hip_cu_count(dev);

@@ -952,14 +952,17 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
     g.strict = m->strict;
     g.hq = m->pf_h;
     g.hsc = m->pf_hs;
-    // the SwiGLU epilogue takes int4 gate/up rows in blocks of 8 + 8, groups of 32 and the 16 x 16 .. 32 x 32
-    // tiles (the shape the gate/up GEMM gets for M tokens)
-    const int gu_shape = pgemm_pick_shape(m->L[0].gu.rows, M, g.simds);
-    const bool fuse_swiglu = m->pf_swiglu && wb == 4 && m->gs == 32 && m->L[0].gu.rb == 16 &&
-                             m->L[0].gu.rows % 64 == 0 && (gu_shape == 11 || gu_shape == 22);
-    // the QKV epilogue takes the 16 x 16 and 32 x 32 tiles
-    const int qkv_shape = pgemm_pick_shape(m->L[0].qkv.rows, M, g.simds);
-    const bool fuse_qkv = m->pf_qkv && (qkv_shape == 11 || qkv_shape == 22);
+    // Tile shapes of the four GEMMs, and with them the layout of each one's input.
+    const Layer &L0 = m->L[0];
+    const bool sw = m->pf_swiglu && wb == 4 && m->gs == 32 && L0.gu.rb == 16 && L0.gu.rows % 64 == 0;
+    const int qkv_shape = pgemm_shape(L0.qkv, M, g.simds, false), o_shape = pgemm_shape(L0.o, M, g.simds, false);
+    const int gu_shape = pgemm_shape(L0.gu, M, g.simds, sw), down_shape = pgemm_shape(L0.down, M, g.simds, false);
+    // the SwiGLU epilogue (sw: int4 gate/up rows in blocks of 8 + 8, groups of 32) takes the 16 x 16 .. 32 x 32 tiles
+    // and k_pgemm32
+    const bool fuse_swiglu = sw && (gu_shape == 11 || gu_shape == 22 || gu_shape == PGEMM_SHAPE_32);
+    // the QKV epilogue takes the 16 x 16 and 32 x 32 tiles and k_pgemm32
+    const bool fuse_qkv = m->pf_qkv && (qkv_shape == 11 || qkv_shape == 22 || qkv_shape == PGEMM_SHAPE_32);
+    g.hlay = down_shape == PGEMM_SHAPE_32;
     PgemmArgs gq = g;
     gq.qkv = 1;
     gq.rope_cos = m->rope_cos;
@@ -976,25 +979,32 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
         pa.vc = m->vc + (size_t)l * m->ctx * kv;
         pa.bias = m->biases ? m->biases + (size_t)l * (dim + 2 * kv) : nullptr;
         pa.norm_w = attn_norm(m, l);
+        pa.lay = qkv_shape == PGEMM_SHAPE_32;
         // after the first layer, the previous down projection's output (in y) joins x before the norm
         HIP_OR_FAIL("llm_prefill", launch_p_norm_quant(pa, l > 0, m->st));
         if (fuse_qkv) {
             gq.W = Ly.qkv;
+            gq.shape = qkv_shape;
             gq.bias = pa.bias;
             gq.kc = pa.kc;
             gq.vc = pa.vc;
             HIP_OR_FAIL("llm_prefill", launch_pgemm(wb, m->gs, sf, gq, m->st));
         } else {
             g.W = Ly.qkv;
+            g.shape = qkv_shape;
             HIP_OR_FAIL("llm_prefill", launch_pgemm(wb, m->gs, sf, g, m->st));
             HIP_OR_FAIL("llm_prefill", launch_p_qkv(pa, m->st));
         }
+        pa.lay = o_shape == PGEMM_SHAPE_32;
         HIP_OR_FAIL("llm_prefill", launch_p_attention(pa, m->st)); // the o projection's int8 input
         g.W = Ly.o;
+        g.shape = o_shape;
         HIP_OR_FAIL("llm_prefill", launch_pgemm(wb, m->gs, sf, g, m->st));
         pa.norm_w = ffn_norm(m, l);
+        pa.lay = gu_shape == PGEMM_SHAPE_32;
         HIP_OR_FAIL("llm_prefill", launch_p_norm_quant(pa, true, m->st)); // x += o output, then the FFN norm
         g.W = Ly.gu;
+        g.shape = gu_shape;
         if (fuse_swiglu) { // h straight from the gate/up GEMM into pf_h, the down GEMM's input
             g.swiglu = 1;
             HIP_OR_FAIL("llm_prefill", launch_pgemm(wb, m->gs, sf, g, m->st));
@@ -1004,9 +1014,11 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
         } else {
             HIP_OR_FAIL("llm_prefill", launch_pgemm(wb, m->gs, sf, g, m->st));
             pa.gu_rb = Ly.gu.rb;
+            pa.lay = down_shape == PGEMM_SHAPE_32;
             HIP_OR_FAIL("llm_prefill", launch_p_swiglu_quant(pa, m->st));
         }
         g.W = Ly.down;
+        g.shape = down_shape;
         HIP_OR_FAIL("llm_prefill", launch_pgemm(wb, m->gs, sf, g, m->st));
         g.xq = m->pf_a;
         g.xs = m->pf_s;

@@ -27,8 +27,24 @@ __host__ __device__ inline size_t pf_scale_off(int m, int g, int MB) {
     return ((size_t)(g >> 2) * MB * 16 + m) * 4 + (g & 3);
 }
 __host__ __device__ inline int pf_blocks(int M) { return (M + 15) / 16; }
-// bytes of the int8 input of n elements (whole chunk pairs) and floats of its scales (whole group quads)
-__host__ __device__ inline size_t pf_act_bytes(int n, int M) { return (size_t)((n / 32 + 1) / 2) * pf_blocks(M) * 1024; }
+// The same input for the GEMM on 32 x 32 tiles (k_pgemm32), whose B slice of a lane is half a chunk: one 1 KiB block
+// per chunk of 32 elements and block of 32 tokens, lane l = 32 h + t with elements 8 h .. 8 h + 7 and 16 + 8 h ..
+// 16 + 8 h + 7 of token t, in quads (4 j .. 4 j + 3, then 16 + 4 j .. 16 + 4 j + 3, for j = 2 h and 2 h + 1: the order
+// in which an int4 segment's dwords j give them).  Blocks are ordered [chunk][token block].
+__host__ __device__ inline size_t pf_act_off32(int m, int k, int M) {
+    const int c = k >> 5, e = k & 31, j = (e & 15) >> 2;
+    return ((size_t)c * ((M + 31) / 32) + (m >> 5)) * 1024 + 16 * (32 * (j >> 1) + (m & 31)) + 8 * (j & 1) +
+           4 * (e >> 4) + (e & 3);
+}
+// where a producer puts element k (its quad at once) of token m: lay 0 the 16-token tiles, 1 the 32-token ones
+__host__ __device__ inline size_t pf_act(int m, int k, int M, int lay) {
+    return lay ? pf_act_off32(m, k, M) : pf_act_off(m, k, pf_blocks(M));
+}
+// bytes of the int8 input of n elements (whole chunk pairs, whole blocks of 32 tokens: either layout fits) and floats
+// of its scales (whole group quads)
+__host__ __device__ inline size_t pf_act_bytes(int n, int M) {
+    return (size_t)((n / 32 + 1) / 2) * ((M + 31) / 32) * 2048;
+}
 __host__ __device__ inline size_t pf_scale_floats(int ng, int M) { return (size_t)((ng + 3) / 4) * pf_blocks(M) * 64; }
 
 struct PgemmArgs {
@@ -38,17 +54,19 @@ struct PgemmArgs {
     float *y;               // [M][d]
     int M;
     int shape;              // 0: pgemm_pick_shape; 10 TA + TB: one wave per 16 TA rows x 16 TB tokens
-                            // (TA 1, 2, 4; TB 1, 2, 4; not 44)
+                            // (TA 1, 2, 4; TB 1, 2, 4; not 44); PGEMM_SHAPE_32: k_pgemm32 (pgemm32_takes), the
+                            // input in the layout of pf_act_off32
     int simds;              // SIMDs of the device (0: 1024)
     // swiglu = 1: W is the gate/up matrix (row-blocks of 16: 8 gate rows, then the 8 matching up rows) and the
     // epilogue writes h = silu(gate) * up quantized (groups of 32, flavour qflavor; strict: the reference
-    // libm's expf) into the token-block tiles hq / hsc instead of y (int4 weights, shapes 11, 12, 21, 22)
-    int swiglu, qflavor, strict;
+    // libm's expf) into the token-block tiles hq / hsc instead of y (int4 weights, shapes 11, 12, 21, 22, PGEMM_SHAPE_32);
+    // hlay: the layout of hq (k_pgemm32's epilogue)
+    int swiglu, qflavor, strict, hlay;
     int8_t *hq;             // pf_act_bytes(rows / 2, M); must not alias xq
     float *hsc;             // pf_scale_floats(rows / 64, M)
     // qkv = 1: W is the fused QKV matrix (rows of q, then k, then v; NeoX: q and k in blocks of 16, 8 rows and
     // their 8 RoPE partners) and the epilogue does k_p_qkv's work with the rows instead of storing y: bias,
-    // RoPE at position p0 + m, q rows to q [M][dim], K and V rows to the layer's caches (shapes 11 and 22)
+    // RoPE at position p0 + m, q rows to q [M][dim], K and V rows to the layer's caches (shapes 11, 22, PGEMM_SHAPE_32)
     int qkv;
     const float *bias;      // [dim + 2 kv_dim] (NeoX) or NULL (interleaved pairs)
     const float *rope_cos, *rope_sin; // [ctx][head_size / 2]
@@ -66,6 +84,22 @@ static inline int pgemm_pick_shape(int d, int M, int simds) {
     return waves22 >= 4L * simds ? 22 : 11;
 }
 
+// k_pgemm32: int4 rows with fp16 scales, records that hold two groups of a row, an even number of groups.
+#define PGEMM_SHAPE_32 32
+static inline bool pgemm32_takes(const TiledMat &W) {
+    return W.wbits == 4 && W.gs == 32 && !W.sf32 && W.rb <= 32 && W.ng % 2 == 0;
+}
+// The shape of one of the model's GEMMs.  k_pgemm32 where it has 7/8 of a wave of 32 rows x 32 tokens per SIMD (measured,
+// k_pgemm's tile / k_pgemm32, us: 0.5B shape, 1024 tokens, o and down, 896 waves: 8.2 / 7.8, 28.6 / 26.4; 512 tokens, 448
+// waves: 6.0 / 7.7, 18.0 / 25.9, QKV, 576 waves: 10.6 / 10.4); with the SwiGLU epilogue 2.25 waves of 64 rows x 32
+// tokens (512 tokens of the 0.5B shape, 2432 waves: 30.9 / 28.1, strict 34.0 / 34.4; 77 of the 7B shape, 1776: 62.6 / 71).
+static inline int pgemm_shape(const TiledMat &W, int M, int simds, bool swiglu) {
+    if (simds <= 0) simds = 1024;
+    const long tiles = (long)((W.rows + 31) / 32) * ((M + 31) / 32);
+    if (pgemm32_takes(W) && (swiglu ? 2 * tiles >= 9L * simds : 8 * tiles >= 7L * simds)) return PGEMM_SHAPE_32;
+    return pgemm_pick_shape(W.rows, M, simds);
+}
+
 struct ProwArgs {           // per-token elementwise kernels
     int M, p0;              // tokens, position of the first one
     int dim, kv_dim, head_size, hidden, gs, qflavor, rope_kind, gu_rb;
@@ -81,7 +115,8 @@ struct ProwArgs {           // per-token elementwise kernels
     const float *rope_cos, *rope_sin; // [ctx][hs/2]
     float *q;               // [M][dim]
     float *kc, *vc;         // this layer's caches [ctx][kv_dim]
-    int8_t *oq;             // quantized output (the next GEMM's input), token-block tiles (pf_act_off)
+    int8_t *oq;             // quantized output (the next GEMM's input), token-block tiles in layout lay (pf_act)
+    int lay;
     float *os;              // its scales (pf_scale_off)
     int n_heads, n_kv;
     int strict;             // 1: reference order (sequential RMSNorm sum, reference-order attention, libm expf)

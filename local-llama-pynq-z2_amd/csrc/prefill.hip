@@ -15,9 +15,10 @@
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-// block_quantize into the token-block tiles of the next GEMM's input (token m of MB blocks)
+// block_quantize into the token-block tiles (layout lay) of the next GEMM's input (token m of M)
 __device__ __forceinline__ void block_quantize_tiles(const float *v, int n, int gs, int flavor, int8_t *q, float *s,
-                                                     int m, int MB) {
+                                                     int m, int M, int lay) {
+    const int MB = pf_blocks(M);
     const int nq = n / 4;
     for (int i0 = 0; i0 < nq; i0 += blockDim.x) {
         const int i = i0 + threadIdx.x;
@@ -25,11 +26,22 @@ __device__ __forceinline__ void block_quantize_tiles(const float *v, int n, int 
         float scale;
         const uint32_t packed = quantize_pack(((const float4 *)v)[ok ? i : 0], gs, flavor, &scale);
         if (ok) {
-            *(uint32_t *)(q + pf_act_off(m, 4 * i, MB)) = packed;
+            *(uint32_t *)(q + pf_act(m, 4 * i, M, lay)) = packed;
             if ((i & (gs / 4 - 1)) == 0) s[pf_scale_off(m, i / (gs / 4), MB)] = scale;
         }
     }
 }
+
+template <int I>
+__device__ __forceinline__ float row_bcast(float x) { // lane I of each row of 16 lanes
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + I, 0xF, 0xF, true));
+}
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
 
 // ------------------------------------------------------------------------------------------------------
 // GEMM: y[m][r] = sum_g ((float)ival(r, m, g) * ws[r][g]) * xs[m][g], groups in order.
@@ -536,9 +548,271 @@ __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
                 const uint32_t b0 = (uint8_t)quant_one(hv[i][j][0], scale, inv, a.qflavor);
                 const uint32_t b1 = (uint8_t)quant_one(hv[i][j][1], scale, inv, a.qflavor);
                 const int k0 = 8 * (tx * TA + i) + 4 * qq + 2 * half;
-                *(uint16_t *)(a.hq + pf_act_off(m, k0, MB)) = (uint16_t)(b0 | (b1 << 8));
+                *(uint16_t *)(a.hq + pf_act(m, k0, a.M, a.hlay)) = (uint16_t)(b0 | (b1 << 8));
             }
             if (w == w0 && q == 0) a.hsc[pf_scale_off(m, (8 * tx * TA) / 32, MB)] = scale;
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------------
+// The same GEMM for many tokens (int4 weights, fp16 scales) on v_mfma_i32_32x32x32_i8: one instruction per group of
+// 32, 32 rows and 32 tokens, tokens as the A operand and weight rows as B, so that lane l of the result holds row
+// l % 32 in all its 16 registers: register 4 i + j is token 8 i + 4 (l / 32) + j.
+//  - the row's scale is one register of the lane, no broadcast through LDS;
+//  - the token's scale is the operand that differs by register and half, but not within a half: lane k of each row of
+//    16 lanes holds token 8 (k / 4) + 4 (l / 32) + k % 4, and register k's multiply takes it as a DPP operand
+//    (row_newbcast:k).  So the products and sums are the 3 instructions per output and group of k_pgemm (the
+//    reference's rounding order, bitwise) and nothing else; FMA (the fast mode) adds the product unrounded: 2.
+//  - weights: lane l loads whole 16-byte segments of row l % 32, of group 2 s in the lower half of the wave and 2 s + 1
+//    in the upper; two v_permlane32_swap leave each group's dwords 2 h, 2 h + 1 in half h, and the nibbles are the
+//    slots of the activation layout (pf_act_off32), which comes in one 16-byte load per lane and group.
+// A wave takes 32 TA rows x 32 tokens, a block 2 x 2 waves (the two in a row share weights, the two in a column
+// activations, through the CU's cache); the next two groups' loads are in flight while two are computed, and each
+// tile's MFMA is issued before the previous tile's products.  Blocks are numbered over groups of 8 token blocks, all
+// row blocks each, and every XCD takes one contiguous eighth (its L2 then serves a few row blocks x 512 tokens).
+//
+// Bound by the vector ALU: of 255 (strict) and 178 (fast) vector instructions per 32 x 32 tile and 4 groups, 192 and
+// 128 are the products and sums, the rest nibbles, scales and lane swaps.  Measured (k_pgemm's tile, then this; fast
+// mode): 512 tokens of the 7B shape, QKV 64.5 -> 42.1 us, o 39.8 -> 30.4, gate/up 312 -> 230 (strict 305), down 196 ->
+// 141; 2000 tokens, gate/up 810 us (strict 1039) for 432 (648) us of products and sums.  Two row tiles per wave for
+// the others: 2000 tokens QKV 109 -> 115, o 82 -> 88, down 409 -> 432 (fewer waves per SIMD).
+template <int EK, int FMA>
+__global__ void __launch_bounds__(256, EK == 1 ? 3 : 4) k_pgemm32(PgemmArgs a) {
+    constexpr int TA = EK == 1 ? 2 : 1; // row tiles per wave (SwiGLU: 32 hidden values, one quantization group)
+    const TiledMat &W = a.W;
+    const int nx = (W.rows + 64 * TA - 1) / (64 * TA), ny = (a.M + 63) / 64, total = nx * ny, per = (total + 7) / 8;
+    const int lin = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || lin >= total) return;
+    const int grp = lin / (8 * nx), rem = lin - grp * 8 * nx, gy = min(8, ny - 8 * grp);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = (2 * (rem / gy) + (w & 1)) * 32 * TA, m0 = (2 * (8 * grp + rem % gy) + (w >> 1)) * 32;
+    if (r0 >= W.rows || m0 >= a.M) return; // the whole wave (no barrier below)
+    const int l = threadIdx.x & 63, l32 = l & 31, l16 = l & 15, h = l >> 5;
+    const int rb = W.rb, gpc = WAVE / rb, lg = 31 - __builtin_clz(gpc), ng = W.ng, ns = ng / 2;
+    const int MB16 = (a.M + 15) >> 4, MB32 = (a.M + 31) >> 5;
+    const uint32_t rstride = (uint32_t)W.nchunks * (uint32_t)W.rec;
+    uint32_t offA[TA], offS[TA];
+#pragma unroll
+    for (int t = 0; t < TA; t++) {
+        const int row = min(r0 + 32 * t + l32, W.rows - 1), bA = row / rb, la = row - bA * rb;
+        offA[t] = bA * rstride + (h * rb + la) * 16;
+        offS[t] = bA * rstride + 1024 + (h * rb + la) * 2;
+    }
+    const uint32_t offB = (uint32_t)(m0 >> 5) * 1024 + 16 * l;
+    const uint32_t offX = (uint32_t)min(m0 + 8 * (l16 >> 2) + 4 * h + (l16 & 3), a.M - 1) * 16;
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)W.data, 0, (int)W.bytes, PG_RSRC3);
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc((void *)a.xq, 0, (int)pf_act_bytes(W.n, a.M), PG_RSRC3);
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)a.xs, 0, (int)(pf_scale_floats(ng, a.M) * 4), PG_RSRC3);
+
+    uint32_t ar[2][TA][4], sr[2][TA];
+    v4i br[2][2];
+    float xr[2][2];
+    auto load = [&](int s, int k) { // groups 2 s, 2 s + 1 into buffer k
+        const int g = 2 * s, c = g >> lg, gi = g & (gpc - 1), so = c * (int)W.rec;
+#pragma unroll
+        for (int t = 0; t < TA; t++) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw, offA[t], so + gi * rb * 16, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) ar[k][t][i] = v[i];
+            sr[k][t] = __builtin_amdgcn_raw_buffer_load_b16(rw, offS[t], so + gi * rb * 2, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(rx, offB, (g + e) * MB32 * 1024, 0);
+            br[k][e] = v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+        }
+        const auto x = __builtin_amdgcn_raw_buffer_load_b64(rs, offX, (g >> 2) * MB16 * 256 + (g & 3) * 4, 0);
+        xr[k][0] = __uint_as_float(x[0]);
+        xr[k][1] = __uint_as_float(x[1]);
+    };
+    v16i magic;
+#pragma unroll
+    for (int i = 0; i < 16; i++) magic[i] = PG_MAGIC_I;
+    float acc[TA][16];
+#pragma unroll
+    for (int t = 0; t < TA; t++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[t][i] = 0.0f;
+    // the tile whose products come next: its MFMA result, the rows' scale, -PG_MAGIC * scale, the tokens' scales
+    v16i d[2];
+    float pw = 0.0f, px = 0.0f;
+    auto products = [&](float (&ac)[16], const v16i &dd, float ws, float xs) {
+        const float nc = -(PG_MAGIC * ws);
+        if constexpr (FMA) {
+#pragma unroll
+            for (int b = 0; b < 16; b += 8) {
+                float p[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) p[i] = fmaf(__int_as_float(dd[b + i]), ws, nc);
+                // ac += xs(token) * p: the compiler has no DPP form for this (it moves xs first); the no-op covers
+                // the two instructions between a vector write of xs and its use as a DPP operand
+#define PG_FMAC8(K0, K1, K2, K3, K4, K5, K6, K7)                                                               \
+                asm("s_nop 1\n\t"                                                                             \
+                    "v_fmac_f32_dpp %0, %8, %9 row_newbcast:" #K0 " row_mask:0xf bank_mask:0xf\n\t"           \
+                    "v_fmac_f32_dpp %1, %8, %10 row_newbcast:" #K1 " row_mask:0xf bank_mask:0xf\n\t"          \
+                    "v_fmac_f32_dpp %2, %8, %11 row_newbcast:" #K2 " row_mask:0xf bank_mask:0xf\n\t"          \
+                    "v_fmac_f32_dpp %3, %8, %12 row_newbcast:" #K3 " row_mask:0xf bank_mask:0xf\n\t"          \
+                    "v_fmac_f32_dpp %4, %8, %13 row_newbcast:" #K4 " row_mask:0xf bank_mask:0xf\n\t"          \
+                    "v_fmac_f32_dpp %5, %8, %14 row_newbcast:" #K5 " row_mask:0xf bank_mask:0xf\n\t"          \
+                    "v_fmac_f32_dpp %6, %8, %15 row_newbcast:" #K6 " row_mask:0xf bank_mask:0xf\n\t"          \
+                    "v_fmac_f32_dpp %7, %8, %16 row_newbcast:" #K7 " row_mask:0xf bank_mask:0xf"              \
+                    : "+v"(ac[b]), "+v"(ac[b + 1]), "+v"(ac[b + 2]), "+v"(ac[b + 3]), "+v"(ac[b + 4]),        \
+                      "+v"(ac[b + 5]), "+v"(ac[b + 6]), "+v"(ac[b + 7])                                       \
+                    : "v"(xs), "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]),   \
+                      "v"(p[7]))
+                if (b == 0) PG_FMAC8(0, 1, 2, 3, 4, 5, 6, 7);
+                else PG_FMAC8(8, 9, 10, 11, 12, 13, 14, 15);
+#undef PG_FMAC8
+            }
+        } else {
+            asm volatile("" : "+v"(xs)); // (one register a tile: shared between row tiles, the broadcasts would be kept in 16)
+            static_for<4>([&](auto b) {
+                float p[4], q[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) p[i] = fmaf(__int_as_float(dd[4 * b.value + i]), ws, nc);
+                static_for<4>([&](auto i) { q[i.value] = row_bcast<4 * b.value + i.value>(xs) * p[i.value]; });
+#pragma unroll
+                for (int i = 0; i < 4; i++) ac[4 * b.value + i] = ac[4 * b.value + i] + q[i];
+            });
+        }
+    };
+    bool first = true;
+    auto step = [&](int k) {
+        float ws[TA][2];
+        uint32_t x[TA][4];
+#pragma unroll
+        for (int t = 0; t < TA; t++) {
+            const auto s02 = __builtin_amdgcn_permlane32_swap(ar[k][t][0], ar[k][t][2], false, false);
+            const auto s13 = __builtin_amdgcn_permlane32_swap(ar[k][t][1], ar[k][t][3], false, false);
+            x[t][0] = s02[0];
+            x[t][1] = s13[0];
+            x[t][2] = s02[1];
+            x[t][3] = s13[1];
+            const uint32_t sv = __float_as_uint(f16_bits_to_f32((uint16_t)sr[k][t]) * 0.0625f);
+            const auto sw = __builtin_amdgcn_permlane32_swap(sv, sv, false, false);
+            ws[t][0] = __uint_as_float(sw[0]);
+            ws[t][1] = __uint_as_float(sw[1]);
+        }
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+#pragma unroll
+            for (int t = 0; t < TA; t++) {
+                const int u = e * TA + t; // unit of the step (2 TA, an even number: parity u & 1)
+                const uint32_t x0 = x[t][2 * e], x1 = x[t][2 * e + 1];
+                const v4i bw = {(int)((x0 << 4) & 0xF0F0F0F0u), (int)(x0 & 0xF0F0F0F0u),
+                                (int)((x1 << 4) & 0xF0F0F0F0u), (int)(x1 & 0xF0F0F0F0u)};
+                d[u & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(br[k][e], bw, magic, 0, 0, 0);
+                if (u > 0 || !first) products(acc[(t + TA - 1) % TA], d[(u & 1) ^ 1], pw, px);
+                pw = ws[t][e];
+                px = xr[k][e];
+            }
+    };
+    load(0, 0);
+    int s = 0;
+    if (ns > 1) {
+        load(1, 1);
+        step(0);
+        first = false;
+        for (s = 1; s + 2 < ns; s += 2) {
+            load(s + 1, 0);
+            step(1);
+            load(s + 2, 1);
+            step(0);
+        }
+        if (s + 1 < ns) { // two left: buffers 1, 0
+            load(s + 1, 0);
+            step(1);
+            step(0);
+        } else {
+            step(1);
+        }
+    } else {
+        step(0);
+    }
+    products(acc[TA - 1], d[1], pw, px);
+
+    if constexpr (EK == 0) {
+#pragma unroll
+        for (int t = 0; t < TA; t++) {
+            const int R = r0 + 32 * t + l32;
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int m = m0 + 8 * (k >> 2) + 4 * h + (k & 3);
+                if (R < W.rows && m < a.M) a.y[(size_t)m * W.rows + R] = acc[t][k];
+            }
+        }
+    } else if constexpr (EK == 2) {
+        // bias, RoPE and the q / K / V writes (k_p_qkv's operations, NeoX pairs): the partner row R ^ 8 is lane l ^ 8
+        const int dim = a.dim, kvd = a.kv_dim, hs = a.head_size, half = hs / 2, rot = dim + kvd, per8 = half / 8;
+#pragma unroll
+        for (int t = 0; t < TA; t++) {
+            const int R = min(r0 + 32 * t + l32, W.rows - 1), blk = R / 16, hh = blk / per8;
+            const int ii = (blk - hh * per8) * 8 + (R & 7);
+            const bool rotated = R < rot, fst = (R & 8) == 0, okr = r0 + 32 * t + l32 < W.rows;
+            const int e = rotated ? hh * hs + (fst ? ii : half + ii) : R, ep = rotated ? hh * hs + (fst ? half + ii : ii) : R;
+            const float bs = a.bias[e], bp = a.bias[ep];
+            float cs[16], sn[16];
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int m = min(m0 + 8 * (k >> 2) + 4 * h + (k & 3), a.M - 1);
+                const size_t o = (size_t)(a.p0 + m) * half + (rotated ? ii : 0);
+                cs[k] = a.rope_cos[o];
+                sn[k] = a.rope_sin[o];
+            }
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int m = m0 + 8 * (k >> 2) + 4 * h + (k & 3), pos = a.p0 + m;
+                const float part = dpp_get<0x128>(acc[t][k]); // row_ror:8, the lane across the halves of the 16
+                const float self = acc[t][k] + bs, partner = part + bp;
+                const float t1 = self * cs[k], t2 = partner * sn[k];
+                const float o = !rotated ? self : fst ? t1 - t2 : t1 + t2;
+                if (okr && m < a.M) {
+                    if (e < dim) a.q[(size_t)m * dim + e] = o;
+                    else if (rotated) a.kc[(size_t)pos * kvd + (e - dim)] = o;
+                    else a.vc[(size_t)pos * kvd + (R - rot)] = o;
+                }
+            }
+        }
+    } else {
+        // SwiGLU (qwen.c:556-562) and int8 quantization of h: a wave's 64 rows are 32 hidden values, one quantization
+        // group: hidden value 16 t + 8 b + v is gate lane 16 b + v, up lane 16 b + 8 + v (of each half) of row tile t.
+        // The gate lanes take the tokens of registers 0 .. 7, the up lanes those of 8 .. 15.
+        const bool up = (l & 8) != 0;
+        float hv[TA][8], gm[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) gm[k] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < TA; t++)
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float own = up ? acc[t][8 + k] : acc[t][k];
+                const float oth = dpp_get<0x128>(up ? acc[t][k] : acc[t][8 + k]);
+                const float g = up ? oth : own, uu = up ? own : oth;
+                const float sig = 1.0f / (1.0f + (a.strict ? ref_expf(-g) : expf(-g)));
+                const float gsg = g * sig;
+                hv[t][k] = gsg * uu;
+                gm[k] = fmaxf(gm[k], fabsf(hv[t][k]));
+            }
+        const int k0 = r0 / 2, g0 = r0 / 64;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            float mx = max8(gm[k]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            const float scale = quant_scale(mx, a.qflavor), inv = quant_inv(scale);
+            const int kk = k + (up ? 8 : 0), m = m0 + 8 * (kk >> 2) + 4 * h + (kk & 3);
+#pragma unroll
+            for (int t = 0; t < TA; t++) {
+                // four lanes' codes in one store, by the first of each four
+                int b = (uint8_t)quant_one(hv[t][k], scale, inv, a.qflavor);
+                b |= __builtin_amdgcn_update_dpp(0, b, 0xF5, 0xF, 0xF, false) << 8; // quad lanes 1, 1, 3, 3
+                b |= __builtin_amdgcn_update_dpp(0, b, 0xAA, 0xF, 0xF, false) << 16; // quad lane 2
+                if ((l & 3) == 0 && m < a.M)
+                    *(uint32_t *)(a.hq + pf_act(m, k0 + 16 * t + 8 * ((l >> 4) & 1) + (l & 7), a.M, a.hlay)) = (uint32_t)b;
+            }
+            if ((l & 23) == 0 && m < a.M) a.hsc[pf_scale_off(m, g0, MB16)] = scale;
         }
     }
 }
@@ -553,7 +827,31 @@ hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStre
     if (W.bytes >= ((size_t)1 << 31) || pf_act_bytes(W.n, a.M) >= ((size_t)1 << 31) ||
         pf_scale_floats(W.ng, a.M) * 4 >= ((size_t)1 << 31))
         return hipErrorInvalidValue;
-    const int shape = a.shape ? a.shape : pgemm_pick_shape(W.rows, a.M, a.simds);
+    const int shape = a.shape ? a.shape : pgemm_pick_shape(W.rows, a.M, a.simds); // (never k_pgemm32: its input differs)
+    if (shape == PGEMM_SHAPE_32) {
+        const int half = a.head_size / 2;
+        if (!pgemm32_takes(W) || wbits != 4 || sf32 || (a.swiglu && a.qkv)) return hipErrorInvalidValue;
+        if (a.swiglu && (W.rb != 16 || W.rows % 64 || !a.hq || !a.hsc || ((uintptr_t)a.hq & 3) || ((uintptr_t)a.hsc & 3)))
+            return hipErrorInvalidValue;
+        if (a.qkv && (W.rows != a.dim + 2 * a.kv_dim || a.head_size % 2 || !a.q || !a.kc || !a.vc || !a.rope_cos ||
+                      !a.rope_sin || a.p0 < 0 || a.rope_kind != ROPE_NEOX || !a.bias ||
+                      (a.dim + a.kv_dim) % 16 || half % 8))
+            return hipErrorInvalidValue;
+        const int br = a.swiglu ? 128 : 64; // rows of a block
+        const long tiles = (long)((W.rows + br - 1) / br) * ((a.M + 63) / 64);
+        const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
+        if (a.swiglu) {
+            if (a.strict) hipLaunchKernelGGL((k_pgemm32<1, 0>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((k_pgemm32<1, 1>), grid, dim3(256), 0, st, a);
+        } else if (a.qkv) {
+            if (a.strict) hipLaunchKernelGGL((k_pgemm32<2, 0>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((k_pgemm32<2, 1>), grid, dim3(256), 0, st, a);
+        } else {
+            if (a.strict) hipLaunchKernelGGL((k_pgemm32<0, 0>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((k_pgemm32<0, 1>), grid, dim3(256), 0, st, a);
+        }
+        return hipGetLastError();
+    }
     const int TA = shape / 10, TB = shape % 10;
     if (a.qkv) {
         // q, k and v rows (NeoX: with the bias, q and k in blocks of 16), shapes 11 and 22
@@ -698,7 +996,7 @@ __global__ void __launch_bounds__(256) k_p_norm_quant(ProwArgs a) {
     }
     for (int i = threadIdx.x + NQ * nt; i < n; i += nt) sv[i] = a.norm_w[i] * (ss * sv[i]);
     __syncthreads();
-    block_quantize_tiles(sv, n, a.gs, a.qflavor, a.oq, a.os, m, pf_blocks(a.M));
+    block_quantize_tiles(sv, n, a.gs, a.qflavor, a.oq, a.os, m, a.M, a.lay);
 }
 
 // QKV rows of token m: bias (qwen.c:521-522), RoPE at position p0 + m (qwen.c:478-488 NeoX pairs; runq.c:506-521
@@ -781,7 +1079,7 @@ __global__ void __launch_bounds__(256) k_p_swiglu_quant(ProwArgs a) {
         }
     }
     __syncthreads();
-    block_quantize_tiles(sv, hid, a.gs, a.qflavor, a.oq, a.os, m, pf_blocks(a.M));
+    block_quantize_tiles(sv, hid, a.gs, a.qflavor, a.oq, a.os, m, a.M, a.lay);
 }
 
 // ------------------------------------------------------------------------------------------------------
@@ -1057,7 +1355,7 @@ __global__ void __launch_bounds__(512) k_p_flash(ProwArgs a, int direct) {
                     const uint32_t b1 = (uint8_t)quant_one(v.y, scale, inv, a.qflavor);
                     const uint32_t b2 = (uint8_t)quant_one(v.z, scale, inv, a.qflavor);
                     const uint32_t b3 = (uint8_t)quant_one(v.w, scale, inv, a.qflavor);
-                    *(uint32_t *)(a.oq + pf_act_off(m, k0 + 16 * (g0 + k), MB)) = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
+                    *(uint32_t *)(a.oq + pf_act(m, k0 + 16 * (g0 + k), a.M, a.lay)) = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
                 }
             if (mine && g == 0) a.os[pf_scale_off(m, (h * HS + 16 * g0) / a.gs, MB)] = scale;
         }
@@ -1176,7 +1474,7 @@ __global__ void __launch_bounds__(256) k_p_attn_merge(ProwArgs a, int all) {
         row[o] = v;
     }
     __syncthreads();
-    block_quantize_tiles(row, a.dim, a.gs, a.qflavor, a.oq, a.os, m, pf_blocks(a.M));
+    block_quantize_tiles(row, a.dim, a.gs, a.qflavor, a.oq, a.os, m, a.M, a.lay);
 }
 
 // Reference-order causal attention: block (h, m) is query head h of token m over positions 0 .. p0 + m
@@ -1212,17 +1510,6 @@ __global__ void __launch_bounds__(256) k_p_attn_strict(ProwArgs a) {
 // one launch 283-308 us for 184 us of multiplies and adds (39.3 T lane operations/s), 980 us before.
 #define SPW_T 64
 __host__ __device__ inline int spw_rows_pad(int M, int kv_mul) { return (M * kv_mul + 15) / 16 * 16; }
-template <int I>
-__device__ __forceinline__ float row_bcast(float x) { // lane I of each row of 16 lanes
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + I, 0xF, 0xF, true));
-}
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
-
 // acc[k] = acc[k] + b_k * x[i][k % VE] for i = 0 .. 15 in order, b_k lane i (of each 16) of w[k / VE]: the products of
 // a few steps first, then their adds, so that no product's register is written again within the two instructions
 // that a DPP operand has to wait for (the compiler fills them with no-ops otherwise).  keep(i, k) false leaves acc[k].
@@ -1453,7 +1740,7 @@ __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) 
         const float scale = quant_scale(gm, a.qflavor), inv = quant_inv(scale);
         if (row0 + r < rows && VE * l < HS) {
             const int k0 = head[r] * HS + VE * l;
-            int8_t *o = a.oq + pf_act_off(tok[r], k0, MB);
+            int8_t *o = a.oq + pf_act(tok[r], k0, a.M, a.lay);
 #pragma unroll
             for (int e = 0; e < VE; e++) o[e] = quant_one(acc[VE * r + e], scale, inv, a.qflavor);
             if ((l & (gl - 1)) == 0) a.os[pf_scale_off(tok[r], k0 / a.gs, MB)] = scale;
@@ -1467,7 +1754,7 @@ __global__ void __launch_bounds__(256) k_p_quant_rows(ProwArgs a) {
     const int m = blockIdx.x, n = a.dim;
     for (int i = threadIdx.x; i < n; i += blockDim.x) sv[i] = a.xb[(size_t)m * n + i];
     __syncthreads();
-    block_quantize_tiles(sv, n, a.gs, a.qflavor, a.oq, a.os, m, pf_blocks(a.M));
+    block_quantize_tiles(sv, n, a.gs, a.qflavor, a.oq, a.os, m, a.M, a.lay);
 }
 
 hipError_t launch_p_embed(const ProwArgs &a, hipStream_t st) {

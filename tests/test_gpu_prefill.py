@@ -11,7 +11,7 @@ import os
 import numpy as np
 import pytest
 
-from helpers import GOLDEN, OracleModel, f16_scales, oracle, pkg, ptr, rel_err, synth
+from helpers import GOLDEN, OracleModel, f16_scales, oracle, pkg, ptr, rel_err, synth, unpack_q4
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3
@@ -69,6 +69,29 @@ def test_prefill_gemm_bit_exact_special_scales(bits, shape):
     xq[4:8] = 127
     xs = rng.uniform(1e-3, 1e-1, size=(M, n // 32)).astype(np.float32)
     check_qwen_gemm(w, s, xq, xs, M, n, d, bits, 16, shape)
+
+
+@pytest.mark.parametrize("M,n,d,rb", [(1, 64, 36, 16), (33, 128, 100, 8), (64, 896, 64, 16), (95, 4864, 160, 8),
+                                      (31, 192, 32, 32), (600, 256, 1152, 16)])
+def test_prefill_gemm32_exact_and_fast(M, n, d, rb):
+    """the 32 x 32 tiles: rows and tokens that fill no tile, one, or end inside one,
+    1 to 76 steps of two groups, records of 2 to 8 groups, special scales in the first rows: bitwise the oracle's in
+    the strict form; the fast form leaves the last product of a term unrounded, so it is held to n/32 roundings of
+    2^-24 of the sum of the terms' magnitudes against float64"""
+    rng = np.random.default_rng(300 + M + n + d)
+    w = rng.integers(0, 256, size=d * n // 2, dtype=np.uint8)
+    w.reshape(d, n // 2)[:8] = 0x88
+    s = f16_scales(rng, d * n // 32, special_rows=1, ng=n // 32)
+    xq = rng.integers(-128, 128, size=(M, n), dtype=np.int8)
+    xq[0] = -128
+    xs = rng.uniform(1e-3, 1e-1, size=(M, n // 32)).astype(np.float32)
+    check_qwen_gemm(w, s, xq, xs, M, n, d, 4, rb, 32)
+    y = pkg().prefill_gemm(w, s, xq, xs, M, n, d, 4, 32, rb, 33)
+    wv = unpack_q4(w, d, n).reshape(d, -1, 32).astype(np.float64) * s.view(np.float16).reshape(d, -1, 1).astype(np.float64)
+    xv = xq.reshape(M, -1, 32).astype(np.float64) * xs[..., None].astype(np.float64)
+    terms = np.einsum("dgk,mgk->mdg", wv, xv)
+    err, size = np.abs(y - terms.sum(2)), np.abs(terms).sum(2)
+    assert (err <= (n // 32 + 1) * 2.0 ** -24 * size).all()
 
 
 @pytest.mark.parametrize("shape", SHAPES)
@@ -182,6 +205,26 @@ def test_prefill_qkv_epilogue_equals_the_separate_kernel(monkeypatch, tmp_path, 
             m.set_strict(True)
         lg = m.prefill(ids)
         runs.append((lg, kv_rows(m, n)))
+        m.close()
+    assert np.array_equal(runs[0][0], runs[1][0])
+    for (ka, va), (kb, vb) in zip(runs[0][1], runs[1][1]):
+        assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+
+
+@pytest.mark.parametrize("strict", [False, True])
+def test_prefill_gemm32_epilogues_equal_the_separate_kernels(monkeypatch, tmp_path, strict):
+    """1100 tokens of the Qwen2-0.5B layer shapes, where every GEMM runs on the 32 x 32 tiles (the last token tile
+    partial): their QKV and SwiGLU epilogues against the plain GEMM and the separate kernels, bitwise"""
+    p = synth("qwb", str(tmp_path / "e32.qwb"), "c3", 61, "layers=2", "vocab=4096", "head_k=4096", "max_seq=1200")
+    ids = [int(v) for v in np.random.default_rng(14).integers(0, 4096, 1100)]
+    runs = []
+    for setting in ("0", "1"):
+        monkeypatch.setenv("LLM_PF_QKV", setting)
+        monkeypatch.setenv("LLM_PF_SWIGLU", setting)
+        m = pkg().Model(p, 1200)
+        m.set_strict(strict)
+        lg = m.prefill(ids)
+        runs.append((lg, kv_rows(m, 1100)))
         m.close()
     assert np.array_equal(runs[0][0], runs[1][0])
     for (ka, va), (kb, vb) in zip(runs[0][1], runs[1][1]):
