@@ -5,6 +5,9 @@
 // order, softmax, weighted sum of V.  Here the softmax is online over sub-chunks of ATT_SUB positions (running
 // max and sum, rescaled partial sums), K and V staged in LDS.
 #pragma once
+#include <type_traits>
+#include <utility>
+
 #include "device.h"
 #include "kernels.h"
 #include "ref_expf.h"
@@ -13,6 +16,42 @@
 #ifndef KERNEL_MARK
 #define KERNEL_MARK(k)
 #endif
+
+template <int I>
+__device__ __forceinline__ float row_bcast(float x) { // lane I of each row of 16 lanes
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + I, 0xF, 0xF, true));
+}
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
+
+// acc[k] = acc[k] + b_k * x[i][k % VE] for i = 0 .. 15 in order, b_k lane i (of each 16) of w[k / VE]: the products of
+// a few steps first, then their adds, so that no product's register is written again within the two instructions
+// that a DPP operand has to wait for (the compiler fills them with no-ops otherwise).  keep(i, k) false leaves acc[k].
+template <int N, int VE, typename K>
+__device__ __forceinline__ void chain16(float (&acc)[N], const float (&w)[N / VE], const float (&x)[16][VE], K &&keep) {
+    constexpr int G = N >= 4 ? 1 : 4 / N; // steps a batch
+    static_for<16 / G>([&](auto b) {
+        float p[G][N];
+        static_for<G>([&](auto g) {
+            constexpr int i = b.value * G + g.value;
+#pragma unroll
+            for (int k = 0; k < N; k++) p[g.value][k] = row_bcast<i>(w[k / VE]) * x[i][k % VE];
+        });
+        __builtin_amdgcn_sched_barrier(0x3f4); // (only vector arithmetic keeps its side of this)
+#pragma unroll
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                const float s = acc[k] + p[g][k];
+                acc[k] = keep(b.value * G + g, k) ? s : acc[k];
+            }
+        __builtin_amdgcn_sched_barrier(0x3f4);
+    });
+}
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 // 16-byte vectors per thread for one sub-chunk of K (and as many of V): ATT_SUB * hs / 4 <= ATT_VEC * 256

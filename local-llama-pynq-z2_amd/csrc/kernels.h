@@ -84,6 +84,8 @@ struct AttnArgs {
     int n_heads, n_kv, hs, kv_dim, splits; // splits: maximum number of position slices (grid)
     int max_pos;            // positions the cache holds (the launcher picks the kernel for the longest slice)
     const StepCtrl *ctrl;
+    float *sc;              // strict mode, long contexts: scores [n_heads][max_pos]
+    int long_ctx;           // 1: the launches for long contexts
 };
 
 struct EmbedArgs {
@@ -157,6 +159,7 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t st);
 // reference-order attention (one block per query head); leaves acc [n_heads][hs] and ml = (0, 1) per head,
 // i.e. the partials of a single slice that the o projection's merge passes through unchanged
 hipError_t launch_attention_strict(const AttnArgs &a, hipStream_t st);
+bool attention_strict_long_ok(const AttnArgs &a); // whether long_ctx has its own launches for this shape
 hipError_t launch_embed(const EmbedArgs &a, hipStream_t st);
 hipError_t launch_argmax(const ArgmaxArgs &a, hipStream_t st);
 hipError_t launch_repack(const RepackArgs &a, hipStream_t st);

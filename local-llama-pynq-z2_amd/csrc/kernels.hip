@@ -925,6 +925,156 @@ __global__ void __launch_bounds__(256) k_attention_strict(AttnArgs a) {
     }
 }
 
+// The same for long contexts, over two launches, so that K and V come through many CUs (one CU draws about 30 GB/s: a
+// head's 3 MB at 3000 positions of head size 128 took k_attention_strict 105 us):
+// k_attn_scores_strict: block = (kv head, tile of 64 positions), the K tile in LDS, lane = position, the kv head's query
+// heads over the waves; a step of the sequential dot is a multiply (the query element a DPP operand) and an add.
+#define ASL_T 64
+template <int HS>
+__global__ void __launch_bounds__(256) k_attn_scores_strict(AttnArgs a) {
+    constexpr int KP = HS + 4, NQ = HS / 16, FV = HS * ASL_T / 1024;
+    __shared__ __align__(16) float kt[ASL_T * KP];
+    const int P = a.ctrl->pos + 1, kvh = blockIdx.x, t0 = ASL_T * blockIdx.y, kv_mul = a.n_heads / a.n_kv;
+    if (t0 >= P) return;
+    const int tid = threadIdx.x, l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const auto rk = __builtin_amdgcn_make_buffer_rsrc((void *)(a.kc + kvh * HS), 0,
+                                                      (int)(((size_t)(P - 1) * a.kv_dim + HS) * 4), 0x00020000);
+#pragma unroll
+    for (int j = 0; j < FV; j++) { // (positions past the last read zeros; their scores are not stored)
+        const int idx = tid + 256 * j, tt = idx / (HS / 4), c = idx - tt * (HS / 4);
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+            rk, t0 + tt < P ? (uint32_t)((t0 + tt) * a.kv_dim + 4 * c) * 4u : 0x80000000u, 0, 0);
+        *(f32x4 *)(kt + tt * KP + 4 * c) = *(const f32x4 *)&v;
+    }
+    float qv[NQ];
+    const int h0 = kvh * kv_mul + min(w, kv_mul - 1);
+#pragma unroll
+    for (int c = 0; c < NQ; c++) qv[c] = a.q[(size_t)h0 * HS + 16 * c + (l & 15)];
+    __syncthreads();
+    const float rs = sqrtf((float)HS);
+    const float *kr = kt + l * KP;
+    for (int j = w; j < kv_mul; j += 4) {
+        const int h = kvh * kv_mul + j;
+        float d[1] = {0.0f};
+#pragma unroll
+        for (int c = 0; c < NQ; c++) {
+            float kk[16][1];
+            const float qc[1] = {qv[c]};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const f32x4 k4 = *(const f32x4 *)(kr + 16 * c + 4 * i);
+                kk[4 * i][0] = k4.x;
+                kk[4 * i + 1][0] = k4.y;
+                kk[4 * i + 2][0] = k4.z;
+                kk[4 * i + 3][0] = k4.w;
+            }
+            chain16<1, 1>(d, qc, kk, [](int, int) { return true; });
+        }
+        if (t0 + l < P) a.sc[(size_t)h * a.max_pos + t0 + l] = d[0] / rs;
+        if (j + 4 < kv_mul) {
+#pragma unroll
+            for (int c = 0; c < NQ; c++) qv[c] = a.q[(size_t)(h + 4) * HS + 16 * c + (l & 15)];
+        }
+    }
+}
+
+// k_attn_values_strict: block = (query head, 16 elements).  Every block of a head computes the head's softmax (max,
+// ref_expf, the sum in position order by block_seq_sum, the division): that is latency, not throughput.  Then waves
+// 1 .. 7 leave the rounded products a_t * v_t[e] of a tile of positions in LDS, V coming four tiles ahead through
+// registers, while wave 0 adds the previous tile in position order, lane = element: its chain is an add per position
+// and a 16-byte LDS read per four, and bounds the kernel (with the softmax sum's chain).  A layer's strict step of the
+// 7B shape at 3000 positions: 170 -> 91 us.
+#define ASL_VT 224  // positions per tile: two 16-byte V vectors per producer thread
+#define ASL_VS 228  // their row stride in LDS (16-byte rows, the 16 lanes' reads spread over the banks)
+#define ASL_VD 4    // tiles in flight
+#define ASL_THREADS 512
+static inline size_t attn_values_lds_bytes(int max_pos) {
+    return ((size_t)(max_pos + 3) / 4 * 4 + 2 * 16 * ASL_VS + 16) * 4 + seq_sum_scratch_bytes(ASL_THREADS) + 16;
+}
+__global__ void __launch_bounds__(ASL_THREADS) k_attn_values_strict(AttnArgs a) {
+    extern __shared__ __align__(16) float sm[];
+    const int P = a.ctrl->pos + 1, h = blockIdx.x, e0 = 16 * blockIdx.y, kv_mul = a.n_heads / a.n_kv;
+    const int tid = threadIdx.x, l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = ASL_THREADS / WAVE;
+    float *at = sm, *pt = at + (a.max_pos + 3) / 4 * 4, *red = pt + 2 * 16 * ASL_VS;
+    uint8_t *scr = (uint8_t *)(red + 16);
+    const auto rv = __builtin_amdgcn_make_buffer_rsrc((void *)(a.vc + (h / kv_mul) * a.hs + e0), 0,
+                                                      (int)(((size_t)(P - 1) * a.kv_dim + 16) * 4), 0x00020000);
+    // producer thread u = tid - 64: vector u % 4 of positions u / 4 and 112 + u / 4 of a tile
+    const int u = max(tid - WAVE, 0), ut = u >> 2, uc = u & 3;
+    f32x4 fr[ASL_VD][2];
+    auto fetch = [&](int kt, f32x4 (&f)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int t = kt * ASL_VT + ut + 112 * j;
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+                rv, w > 0 && t < P ? (uint32_t)(t * a.kv_dim + 4 * uc) * 4u : 0x80000000u, 0, 0);
+            f[j] = *(const f32x4 *)&v;
+        }
+    };
+    // scores and their maximum
+    const float *sc = a.sc + (size_t)h * a.max_pos;
+    float mx = -INFINITY;
+    for (int i = 0; i < P; i += 8 * ASL_THREADS) {
+        float s[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) s[k] = sc[min(i + k * ASL_THREADS + tid, P - 1)];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int t = i + k * ASL_THREADS + tid;
+            if (t < P) at[t] = s[k];
+            mx = fmaxf(mx, s[k]);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < ASL_VD; d++) fetch(d, fr[d]);
+    mx = wave_max(mx);
+    if (l == 0) red[w] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < nw; k++) mx = fmaxf(mx, red[k]);
+    for (int t = tid; t < P; t += ASL_THREADS) at[t] = ref_expf(at[t] - mx);
+    __syncthreads();
+    const float sum = block_seq_sum(at, P, scr);
+    __syncthreads(); // every wave's walk may still read the exponentials that the division below overwrites
+    for (int t = tid; t < P; t += ASL_THREADS) at[t] = at[t] / sum;
+    __syncthreads();
+    const int nt = (P + ASL_VT - 1) / ASL_VT;
+    float acc = 0.0f;
+    for (int k0 = 0; k0 <= nt; k0 += ASL_VD)
+#pragma unroll
+        for (int d = 0; d < ASL_VD; d++) {
+            const int kt = k0 + d;
+            if (kt > nt) break;
+            if (w == 0) {
+                if (kt > 0) acc = seq_chain(acc, pt + ((kt - 1) & 1) * 16 * ASL_VS + (l & 15) * ASL_VS, 0, ASL_VT);
+            } else if (kt < nt) {
+                float *o = pt + (kt & 1) * 16 * ASL_VS + 4 * uc * ASL_VS;
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const int tt = ut + 112 * j, t = kt * ASL_VT + tt;
+                    const float p = at[min(t, P - 1)];
+                    const f32x4 v = fr[d][j];
+                    // (+0 past the last position: it leaves the sum, which is never -0, unchanged)
+                    o[tt] = t < P ? p * v.x : 0.0f;
+                    o[ASL_VS + tt] = t < P ? p * v.y : 0.0f;
+                    o[2 * ASL_VS + tt] = t < P ? p * v.z : 0.0f;
+                    o[3 * ASL_VS + tt] = t < P ? p * v.w : 0.0f;
+                }
+                fetch(kt + ASL_VD, fr[d]);
+            }
+            __syncthreads();
+        }
+    if (tid < 16) a.acc[(size_t)h * a.hs + e0 + tid] = acc;
+    if (tid == 0 && blockIdx.y == 0) {
+        a.ml[2 * h] = 0.0f;
+        a.ml[2 * h + 1] = 1.0f;
+    }
+}
+
+bool attention_strict_long_ok(const AttnArgs &a) {
+    return a.sc && (a.hs == 32 || a.hs == 48 || a.hs == 64 || a.hs == 128) && attn_values_lds_bytes(a.max_pos) <= 65536;
+}
+
 hipError_t launch_attention_strict(const AttnArgs &a, hipStream_t st) {
     const size_t lds = attn_strict_lds_floats(a.hs, a.max_pos, 256) * 4;
     // the K and V reads go through buffer resources: a layer's cache must stay below 2 GiB
@@ -932,6 +1082,15 @@ hipError_t launch_attention_strict(const AttnArgs &a, hipStream_t st) {
         a.n_heads % a.n_kv ||
         (size_t)(a.max_pos + 64) * a.kv_dim * 4 >= 0x7fffffffu)
         return hipErrorInvalidValue;
+    if (a.long_ctx && attention_strict_long_ok(a)) {
+        const dim3 gs(a.n_kv, (a.max_pos + ASL_T - 1) / ASL_T), gv(a.n_heads, a.hs / 16);
+        if (a.hs == 32) hipLaunchKernelGGL(k_attn_scores_strict<32>, gs, dim3(256), 0, st, a);
+        else if (a.hs == 48) hipLaunchKernelGGL(k_attn_scores_strict<48>, gs, dim3(256), 0, st, a);
+        else if (a.hs == 64) hipLaunchKernelGGL(k_attn_scores_strict<64>, gs, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL(k_attn_scores_strict<128>, gs, dim3(256), 0, st, a);
+        hipLaunchKernelGGL(k_attn_values_strict, gv, dim3(ASL_THREADS), attn_values_lds_bytes(a.max_pos), st, a);
+        return hipGetLastError();
+    }
     if (a.hs == 64) hipLaunchKernelGGL(k_attention_strict<64>, dim3(a.n_heads), dim3(256), lds, st, a);
     else if (a.hs == 128) hipLaunchKernelGGL(k_attention_strict<128>, dim3(a.n_heads), dim3(256), lds, st, a);
     else hipLaunchKernelGGL(k_attention_strict<0>, dim3(a.n_heads), dim3(256), lds, st, a);

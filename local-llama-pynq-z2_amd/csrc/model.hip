@@ -78,13 +78,15 @@ struct llm_model {
     int32_t *head_ids_d = nullptr;
     std::vector<int32_t> head_ids_h;
     float *kc = nullptr, *vc = nullptr, *x = nullptr, *q = nullptr, *att_ml = nullptr, *att_acc = nullptr;
+    float *att_sc = nullptr; // strict mode: scores [n_heads][ctx]
     float *logits = nullptr, *hist = nullptr, *part_v = nullptr, *hsc = nullptr;
     int8_t *hq = nullptr;
     int *part_i = nullptr;
     int part_cap = 0; // argmax partials allocated (the larger head grid of the two modes)
     StepCtrl *ctrl = nullptr;
     int *prompt = nullptr, *tokens = nullptr, *gen = nullptr;
-    hipGraphExec_t g_plain = nullptr, g_hist = nullptr;
+    // captured steps: [0 decode, 1 keeping every position's logits][sampled][0 short, 1 long contexts] (step_graph)
+    hipGraphExec_t g_step[2][2][2] = {};
     // on-device sampler (temperature > 0): settings and RNG on the device, scratch, the sampling step graphs
     bool sampling = false;
     SamplerState *ss = nullptr;
@@ -92,7 +94,6 @@ struct llm_model {
     void *smp_scratch = nullptr; // the many-workgroup draw's buffers (large vocabularies)
     void *smp_strict = nullptr;  // the reference-order draw's buffers (strict mode)
     int smp_path = -1;           // top-p (1) or the plain walk (0): the sampled step graphs launch that path only
-    hipGraphExec_t g_plain_s = nullptr, g_hist_s = nullptr;
     // prefill: activation matrices of up to pf_cap tokens (allocated on first use)
     int pf_cap = 0, prefill_on = 1;
     float *pf_x = nullptr, *pf_y = nullptr, *pf_q = nullptr, *pf_s = nullptr;
@@ -218,13 +219,19 @@ hipError_t launch_sampler(llm_model *m) {
     return launch_sample(a, m->st);
 }
 
+// Whether the step at `pos` takes the launches for long contexts (both kinds are right at any position).  Strict, from
+// 192 positions (a layer's step, one kernel per head / scores and values apart, us: 7B shape 160 positions 73.1 / 73.0,
+// 256 78.0 / 75.5, 3000 170 / 91; 0.5B shape 160 36.8 / 38.0, 256 39.9 / 39.0, 3000 98 / 52; llama2.c 768 160 34.1 /
+// 34.2, 256 37.1 / 35.1; 288 96 30.8 / 31.3, 160 32.4 / 31.7).
+bool long_step(const llm_model *m, int pos) { return m->strict && pos + 1 >= 192; }
+
 // Enqueue one decode step on m->st.  prof != NULL records events around every launch.  Kernel kinds whose
 // bit is set in `skip` are left out (the in-graph timing of llm_profile_graph compares such steps).  With
 // `sampled`, the sampler follows the head.
 int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finalize, unsigned skip = 0,
                  bool sampled = false) {
     const llm_info &I = m->info;
-    const int dim = I.dim, kv = m->kv_dim;
+    const int dim = I.dim, kv = m->kv_dim, lng = long_step(m, pos_hint);
     auto mark = [&](int kind, double bytes) {
         if (!prof) return;
         if (prof->used + 2 > prof->ev.size()) {
@@ -305,6 +312,8 @@ int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finaliz
         t.splits = m->att_splits;
         t.max_pos = m->ctx;
         t.ctrl = m->ctrl;
+        t.sc = m->att_sc;
+        t.long_ctx = lng;
         if (on(K_ATTN)) {
             mark(K_ATTN, kind_bytes(m, K_ATTN, pos_hint));
             if (m->strict) {
@@ -367,10 +376,11 @@ int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finaliz
     return 0;
 }
 
-int capture(llm_model *m, bool hist, hipGraphExec_t *out, unsigned skip = 0, bool sampled = false) {
+// the step at position pos (its kind of launches) as a graph, which serves any position
+int capture(llm_model *m, bool hist, hipGraphExec_t *out, int pos, unsigned skip = 0, bool sampled = false) {
     hipGraph_t g;
     HIP_OR_FAIL("llm", hipStreamBeginCapture(m->st, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_step(m, hist, nullptr, 0, false, skip, sampled);
+    int rc = enqueue_step(m, hist, nullptr, pos, false, skip, sampled);
     hipError_t e = hipStreamEndCapture(m->st, &g);
     if (rc || e != hipSuccess) {
         fprintf(stderr, "llm: graph capture failed: %s\n", hipGetErrorString(e));
@@ -383,6 +393,23 @@ int capture(llm_model *m, bool hist, hipGraphExec_t *out, unsigned skip = 0, boo
         return -1;
     }
     return 0;
+}
+
+// the captured step for position pos, captured at its first use; NULL (message printed) on failure
+hipGraphExec_t step_graph(llm_model *m, bool hist, bool sampled, int pos) {
+    hipGraphExec_t *g = &m->g_step[hist][sampled][long_step(m, pos)];
+    if (!*g && capture(m, hist, g, pos, 0, sampled)) return nullptr;
+    return *g;
+}
+
+void drop_graphs(llm_model *m, bool sampled_only) {
+    for (auto &of_hist : m->g_step)
+        for (int smp = sampled_only ? 1 : 0; smp < 2; smp++)
+            for (hipGraphExec_t &g : of_hist[smp])
+                if (g) {
+                    hipGraphExecDestroy(g);
+                    g = nullptr;
+                }
 }
 
 int set_ctrl(llm_model *m, int pos, int token, int n_prompt, int mode) {
@@ -516,6 +543,7 @@ int finish_setup(llm_model *m) {
         dalloc(m, &m->q, (size_t)I.dim * 4) ||
         dalloc(m, &m->att_ml, (size_t)I.n_heads * m->att_splits * 2 * 4) ||
         dalloc(m, &m->att_acc, (size_t)I.n_heads * m->att_splits * m->hs * 4) ||
+        dalloc(m, &m->att_sc, (size_t)I.n_heads * m->ctx * 4) ||
         dalloc(m, &m->logits, (size_t)I.n_logits * 4) || dalloc(m, &m->part_v, (size_t)head_grid * 4) ||
         dalloc(m, &m->part_i, (size_t)head_grid * 4) || dalloc(m, &m->hq, (size_t)I.hidden_dim) ||
         dalloc(m, &m->hsc, (size_t)I.hidden_dim / m->gs * 4) || dalloc(m, &m->ctrl, sizeof(StepCtrl)) ||
@@ -1050,8 +1078,7 @@ int prefill_all(llm_model *m, const int *ids, int n, bool sampled = false, int p
 
 void free_model(llm_model *m) {
     if (m->st) hipStreamSynchronize(m->st);
-    for (hipGraphExec_t g : {m->g_plain, m->g_hist, m->g_plain_s, m->g_hist_s})
-        if (g) hipGraphExecDestroy(g);
+    drop_graphs(m, false);
     for (void *p : m->allocs) hipFree(p);
     if (m->hist) hipFree(m->hist);
     for (void *p : {(void *)m->pf_x, (void *)m->pf_y, (void *)m->pf_q, (void *)m->pf_s,
@@ -1168,14 +1195,18 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
         }
     hipSetDevice(m->device);
     const bool hist = logits != nullptr, smp = m->sampling;
-    hipGraphExec_t *g = smp ? (hist ? &m->g_hist_s : &m->g_plain_s) : (hist ? &m->g_hist : &m->g_plain);
     if (hist && !m->hist) {
         if (hipMalloc(&m->hist, (size_t)m->ctx * m->info.n_logits * 4) != hipSuccess) {
             fprintf(stderr, "llm_generate: no room for the logits history\n");
             return -1;
         }
     }
-    if (!*g && capture(m, hist, g, 0, smp)) return -1;
+    auto launch = [&](int pos) -> int {
+        hipGraphExec_t g = step_graph(m, hist, smp, pos);
+        if (!g) return -1;
+        HIP_OR_FAIL("llm_generate", hipGraphLaunch(g, m->st));
+        return 0;
+    };
     HIP_OR_FAIL("llm_generate", hipMemcpy(m->prompt + pos0, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice));
     const int end_prompt = pos0 + n_prompt; // positions below take their token from the prompt
     if (set_ctrl(m, pos0 - 1, 0, end_prompt, 1)) return -1;
@@ -1187,7 +1218,8 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
         if (prefill_all(m, prompt, n_prompt, smp, pos0)) return -1;
         if (set_ctrl(m, end_prompt - 1, prompt[n_prompt - 1], end_prompt, 1)) return -1;
     } else {
-        for (int p = 0; p < n_prompt; p++) HIP_OR_FAIL("llm_generate", hipGraphLaunch(*g, m->st));
+        for (int p = 0; p < n_prompt; p++)
+            if (launch(pos0 + p)) return -1;
     }
     HIP_OR_FAIL("llm_generate", hipStreamSynchronize(m->st));
     const double t1 = now_ms();
@@ -1199,7 +1231,8 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
     bool done = false;
     while (!done) {
         const int upto = ran + batch < last_pos ? ran + batch : last_pos;
-        for (int p = ran + 1; p <= upto; p++) HIP_OR_FAIL("llm_generate", hipGraphLaunch(*g, m->st));
+        for (int p = ran + 1; p <= upto; p++)
+            if (launch(p)) return -1;
         ran = upto > ran ? upto : ran;
         HIP_OR_FAIL("llm_generate", launch_finalize(m)); // argmax of the batch's last step
         HIP_OR_FAIL("llm_generate", hipMemcpyAsync(gen.data() + checked, m->gen + checked,
@@ -1254,13 +1287,14 @@ extern "C" int llm_decode_replay(llm_model *m, int steps, double *ms) {
     c.mode = 1;
     c.n_prompt = 0;
     HIP_OR_FAIL("llm_decode_replay", hipMemcpy(m->ctrl, &c, sizeof c, hipMemcpyHostToDevice));
-    hipGraphExec_t *g = m->sampling ? &m->g_plain_s : &m->g_plain;
-    if (!*g && capture(m, false, g, 0, m->sampling)) return -1;
+    std::vector<hipGraphExec_t> g(steps); // (captured before the clock starts)
+    for (int i = 0; i < steps; i++)
+        if (!(g[i] = step_graph(m, false, m->sampling, c.pos + 1 + i))) return -1;
     hipEvent_t e0, e1;
     hipEventCreate(&e0);
     hipEventCreate(&e1);
     hipEventRecord(e0, m->st);
-    for (int i = 0; i < steps; i++) HIP_OR_FAIL("llm_decode_replay", hipGraphLaunch(*g, m->st));
+    for (int i = 0; i < steps; i++) HIP_OR_FAIL("llm_decode_replay", hipGraphLaunch(g[i], m->st));
     hipEventRecord(e1, m->st);
     HIP_OR_FAIL("llm_decode_replay", hipEventSynchronize(e1));
     float t = 0;
@@ -1338,8 +1372,8 @@ extern "C" int llm_profile_graph(llm_model *m, int steps, int rounds, llm_kernel
     const int per_step[] = {1, m->info.n_layers, m->info.n_layers, m->info.n_layers, m->info.n_layers,
                             m->info.n_layers, 1};
     std::vector<hipGraphExec_t> g(nk + 1, nullptr);
-    int rc = capture(m, false, &g[nk]);
-    for (int k = 0; k < nk && !rc; k++) rc = capture(m, false, &g[k], 1u << kinds[k]);
+    int rc = capture(m, false, &g[nk], c.pos + 1);
+    for (int k = 0; k < nk && !rc; k++) rc = capture(m, false, &g[k], c.pos + 1, 1u << kinds[k]);
     hipEvent_t e0, e1;
     hipEventCreate(&e0);
     hipEventCreate(&e1);
@@ -1441,11 +1475,7 @@ extern "C" int llm_set_sampler(llm_model *m, float temperature, float topp, unsi
     // the sampled step graphs hold one path's launches: captured again when the other one is set
     const int path = topp > 0.0f && topp < 1.0f ? 1 : 0;
     if (path != m->smp_path) {
-        for (hipGraphExec_t *g : {&m->g_plain_s, &m->g_hist_s})
-            if (*g) {
-                hipGraphExecDestroy(*g);
-                *g = nullptr;
-            }
+        drop_graphs(m, true);
         m->smp_path = path;
     }
     return 0;
@@ -1473,11 +1503,7 @@ extern "C" int llm_set_strict(llm_model *m, int on) {
         return -1;
     }
     // the captured step graphs hold the other mode's kernels and shapes
-    for (hipGraphExec_t *g : {&m->g_plain, &m->g_hist, &m->g_plain_s, &m->g_hist_s})
-        if (*g) {
-            hipGraphExecDestroy(*g);
-            *g = nullptr;
-        }
+    drop_graphs(m, false);
     return 0;
 }
 

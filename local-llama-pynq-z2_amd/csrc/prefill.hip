@@ -32,17 +32,6 @@ __device__ __forceinline__ void block_quantize_tiles(const float *v, int n, int 
     }
 }
 
-template <int I>
-__device__ __forceinline__ float row_bcast(float x) { // lane I of each row of 16 lanes
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + I, 0xF, 0xF, true));
-}
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
-
 // ------------------------------------------------------------------------------------------------------
 // GEMM: y[m][r] = sum_g ((float)ival(r, m, g) * ws[r][g]) * xs[m][g], groups in order.
 //
@@ -1510,31 +1499,6 @@ __global__ void __launch_bounds__(256) k_p_attn_strict(ProwArgs a) {
 // one launch 283-308 us for 184 us of multiplies and adds (39.3 T lane operations/s), 980 us before.
 #define SPW_T 64
 __host__ __device__ inline int spw_rows_pad(int M, int kv_mul) { return (M * kv_mul + 15) / 16 * 16; }
-// acc[k] = acc[k] + b_k * x[i][k % VE] for i = 0 .. 15 in order, b_k lane i (of each 16) of w[k / VE]: the products of
-// a few steps first, then their adds, so that no product's register is written again within the two instructions
-// that a DPP operand has to wait for (the compiler fills them with no-ops otherwise).  keep(i, k) false leaves acc[k].
-template <int N, int VE, typename K>
-__device__ __forceinline__ void chain16(float (&acc)[N], const float (&w)[N / VE], const float (&x)[16][VE], K &&keep) {
-    constexpr int G = N >= 4 ? 1 : 4 / N; // steps a batch
-    static_for<16 / G>([&](auto b) {
-        float p[G][N];
-        static_for<G>([&](auto g) {
-            constexpr int i = b.value * G + g.value;
-#pragma unroll
-            for (int k = 0; k < N; k++) p[g.value][k] = row_bcast<i>(w[k / VE]) * x[i][k % VE];
-        });
-        __builtin_amdgcn_sched_barrier(0x3f4); // (only vector arithmetic keeps its side of this)
-#pragma unroll
-        for (int g = 0; g < G; g++)
-#pragma unroll
-            for (int k = 0; k < N; k++) {
-                const float s = acc[k] + p[g][k];
-                acc[k] = keep(b.value * G + g, k) ? s : acc[k];
-            }
-        __builtin_amdgcn_sched_barrier(0x3f4);
-    });
-}
-
 template <int HS, int R>
 __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) {
     constexpr int KP = HS + 4, NQ = HS / 16, VE = HS > 64 ? 2 : 1, FV = HS * SPW_T / 1024;

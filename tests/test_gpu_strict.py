@@ -19,7 +19,7 @@ import os
 import numpy as np
 import pytest
 
-from helpers import GOLDEN, REF_DIR, oracle, pkg, ptr, synth
+from helpers import GOLDEN, REF_DIR, OracleModel, oracle, pkg, ptr, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -277,4 +277,28 @@ def test_strict_runq_full_context(tmp_path, preset, seed):
     m.set_strict(True)
     r = m.generate(prompt, steps - len(prompt) + 1, logits=True)
     check_bitwise(m, ref, r["ids"], r["logits"], ids_r, lg_r, len(lg_r))
+    m.close()
+
+
+@pytest.mark.parametrize("fmt,shape", [("qwb", ("dim=512", "heads=4", "kv_heads=1")),
+                                       ("qwb", ("dim=384", "heads=8", "kv_heads=8")),
+                                       ("qwb", ("dim=256", "heads=8", "kv_heads=2")),
+                                       ("qwb", ("dim=1024", "heads=16", "kv_heads=1")),
+                                       ("bin", ("dim=192", "heads=4", "kv_heads=2"))])
+def test_strict_long_context_decode_equals_the_oracle(tmp_path, fmt, shape):
+    """decode steps through position 469, across the switch to the long-context attention (192 positions), its score
+    tiles of 64 and its value tiles of 224 positions, head sizes 128, 48, 32 and 64, 1 to 16 query heads per kv head:
+    every position's logits bit for bit, eager steps and the captured ones (both kinds of graph in one generation)"""
+    n = 470
+    extra = ["hidden=256", "layers=2", "vocab=512", "max_seq=500"] + (["head_k=256"] if fmt == "qwb" else [])
+    p = synth(fmt, str(tmp_path / f"l.{fmt}"), "tiny", 9, *shape, *extra)
+    m, om = pkg().Model(p, 500), OracleModel(p, 500)
+    m.set_strict(True)
+    ids = [int(om.head_ids[v]) for v in np.random.default_rng(3).integers(2, om.n, n)]
+    ref = np.stack([om.forward(t, pos) for pos, t in enumerate(ids)])
+    om.close()
+    for pos, t in enumerate(ids):
+        assert np.array_equal(m.forward(t, pos), ref[pos]), pos
+    m.set_prefill(False)
+    assert np.array_equal(m.generate(ids, 1, logits=True)["logits"], ref)
     m.close()
