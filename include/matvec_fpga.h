@@ -9,8 +9,9 @@
  *   - the weight and scale ranges (w/wq, ws) are copied to HBM the first time they are used as weights and
  *     then kept resident (repacked once into the GEMV kernels' tiled layout); the reference's callers write
  *     weights once at load (qwen.c:162-163, runq.c:167-168) and never again,
- *   - the activation ranges (xq, xs) are copied host->device on every call,
- *   - the output range is copied device->host before the call returns.
+ *   - the activation ranges (xq, xs) are read from the host buffer on every call,
+ *   - the output range of the host buffer is written before the call returns (the HBM twin of an output range is
+ *     not: no call reads it).
  * Calls are synchronous, like the reference's (run_kernel polls ap_done, matvec_fpga.cpp:156-170).  State is
  * process-global and not thread-safe, like the reference's (its file-scope state, matvec_fpga.cpp:50-56).
  *

@@ -17,8 +17,14 @@ namespace {
 
 struct Buf {
     uint8_t *host, *dev;
+    uint8_t *hdev; // the host buffer's address on the device (pinned host memory, which kernels read and write)
     size_t size;
 };
+
+// A call's end for the host that spins on it: the store follows every store of the kernels before it in the stream.
+__global__ void k_done(uint32_t *flag, uint32_t seq) {
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 struct Weight { // one matrix, uploaded and repacked at its first use
     uint8_t *tiled;
@@ -39,10 +45,12 @@ struct State {
     size_t total = 0;
     char last_err[256] = "";
     uint8_t *stage = nullptr;    // int rowmap for repacks
-    int8_t *xstage = nullptr;    // activations whose device address is not 16-byte aligned (the kernel reads
-                                 // them as 16-byte vectors)
-    float *sstage = nullptr;     // activation scales whose device address is not 4-byte aligned
-    float *ostage = nullptr;     // outputs whose device address is not 4-byte aligned
+    int8_t *xstage = nullptr;    // activations whose address is not 16-byte aligned (the kernel reads them as
+                                 // 16-byte vectors)
+    float *sstage = nullptr;     // activation scales whose address is not 4-byte aligned
+    float *ostage = nullptr;     // outputs whose address is not 4-byte aligned
+    uint32_t *done = nullptr, *done_dev = nullptr; // pinned word: the last finished call (k_done)
+    uint32_t seq = 0;            // the last started one
     size_t ostage_n = 0;
     int strict = 0;              // LLM_STRICT=1: fpga_matvec4 adds a row's groups in order (qwen.c:452-455)
     int *rowmap = nullptr;
@@ -121,23 +129,41 @@ const Weight *weight(const char *who, uint64_t w, uint64_t ws, int n, int d, int
     return &S.weights.emplace(key, x).first->second;
 }
 
+// Whether the call finishes within a millisecond (the stream's own queries, which cost about 15 us each, and sleeps
+// are for the calls that do not).
+bool spin_done() {
+    struct timespec t0, t;
+    clock_gettime(CLOCK_MONOTONIC, &t0);
+    for (;;) {
+        for (int i = 0; i < (S.timeout_ms < 1 ? 1 : 256); i++)
+            if (__atomic_load_n(S.done, __ATOMIC_ACQUIRE) == S.seq) return true;
+        if (S.timeout_ms < 1) return false;
+        clock_gettime(CLOCK_MONOTONIC, &t);
+        if ((t.tv_sec - t0.tv_sec) * 1000000000L + (t.tv_nsec - t0.tv_nsec) > 1000000L) return false;
+    }
+}
+
 int run(const char *who, const Weight *W, uint64_t xq, uint64_t xs, uint64_t out, int n, int d, int gs) {
     const Buf *bx = find(xq, (size_t)n), *bxs = find(xs, (size_t)(n / gs) * 4), *bo = find(out, (size_t)d * 4);
     if (!bx || !bxs || !bo) {
         fprintf(stderr, "%s: xq, xs or out range is not inside a buffer from fpga_alloc()\n", who);
         return -1;
     }
-    int8_t *xdev = (int8_t *)xq;
+    // The GEMV reads the call's activations from pinned host memory and stores its outputs there: no copy command before
+    // or after it (a call was bound by its two copies in, one out and the wait: 57-89 us at 288 x 288 to 65536 x 896; a
+    // launch that brings the activations to HBM first 14-26 us, this 12-23).  Ranges at addresses that the kernel cannot read or write as aligned vectors go through aligned
+    // device buffers (the reference's driver takes any address for fpga_matvec).
+    int8_t *xdev = (int8_t *)(bx->hdev + (xq - (uint64_t)bx->dev));
+    float *sdev = (float *)(bxs->hdev + (xs - (uint64_t)bxs->dev)), *odev = (float *)(bo->hdev + (out - (uint64_t)bo->dev));
     if (xq & 15) {
         if (!S.xstage) HIP_OR_FAIL(who, hipMalloc(&S.xstage, MATVEC_HIP_MAX_N));
         xdev = S.xstage;
+        HIP_OR_FAIL(who, hipMemcpyAsync(xdev, host_of(bx, xq), (size_t)n, hipMemcpyHostToDevice, S.st));
     }
-    // the kernel reads the scales and writes the outputs as floats: ranges at addresses that are not 4-byte
-    // aligned go through aligned staging buffers (the reference's driver takes any address for fpga_matvec)
-    float *sdev = (float *)xs, *odev = (float *)out;
     if (xs & 3) {
         if (!S.sstage) HIP_OR_FAIL(who, hipMalloc(&S.sstage, MATVEC_HIP_MAX_N / 32 * 4));
         sdev = S.sstage;
+        HIP_OR_FAIL(who, hipMemcpyAsync(sdev, host_of(bxs, xs), (size_t)(n / gs) * 4, hipMemcpyHostToDevice, S.st));
     }
     if (out & 3) {
         if ((size_t)d > S.ostage_n) {
@@ -149,8 +175,6 @@ int run(const char *who, const Weight *W, uint64_t xq, uint64_t xs, uint64_t out
         }
         odev = S.ostage;
     }
-    HIP_OR_FAIL(who, hipMemcpyAsync(xdev, host_of(bx, xq), (size_t)n, hipMemcpyHostToDevice, S.st));
-    HIP_OR_FAIL(who, hipMemcpyAsync(sdev, host_of(bxs, xs), (size_t)(n / gs) * 4, hipMemcpyHostToDevice, S.st));
     GemvArgs a;
     memset(&a, 0, sizeof a);
     a.W = W->T;
@@ -162,10 +186,12 @@ int run(const char *who, const Weight *W, uint64_t xq, uint64_t xs, uint64_t out
     a.xs = sdev;
     a.out = odev;
     HIP_OR_FAIL(who, launch_gemv(W->T.wbits, W->T.gs, W->T.sf32, PRO_XQ, EPI_STORE, a, W->shape.grid, S.st));
-    if (odev != (float *)out) // keep the twin equal to the host copy
-        HIP_OR_FAIL(who, hipMemcpyAsync((void *)out, odev, (size_t)d * 4, hipMemcpyDeviceToDevice, S.st));
-    HIP_OR_FAIL(who, hipMemcpyAsync(host_of(bo, out), odev, (size_t)d * 4, hipMemcpyDeviceToHost, S.st));
-    int r = stream_wait(S.st, S.timeout_ms, who);
+    if (out & 3) HIP_OR_FAIL(who, hipMemcpyAsync(host_of(bo, out), odev, (size_t)d * 4, hipMemcpyDeviceToHost, S.st));
+    S.seq++;
+    hipLaunchKernelGGL(k_done, dim3(1), dim3(1), 0, S.st, S.done_dev, S.seq);
+    HIP_OR_FAIL(who, hipGetLastError());
+    if (spin_done()) return 0;
+    int r = S.timeout_ms < 1 ? 1 : stream_wait(S.st, S.timeout_ms, who); // (a limit of 0: one look)
     if (r == 1) {
         fprintf(stderr, "%s: kernel did not finish in %ld ms (n=%d d=%d)\n", who, S.timeout_ms, n, d);
         return -1;
@@ -187,6 +213,9 @@ int open_impl() {
     }
     HIP_OR_FAIL("fpga", hipSetDevice(dev));
     HIP_OR_FAIL("fpga", hipStreamCreateWithFlags(&S.st, hipStreamNonBlocking));
+    HIP_OR_FAIL("fpga", hipHostMalloc((void **)&S.done, sizeof(uint32_t), hipHostMallocCoherent | hipHostMallocMapped));
+    HIP_OR_FAIL("fpga", hipHostGetDevicePointer((void **)&S.done_dev, S.done, 0));
+    *S.done = S.seq = 0;
     S.device = dev;
     if (const char *e = getenv("FPGA_TIMEOUT_MS")) {
         char *end;
@@ -220,7 +249,9 @@ extern "C" void *fpga_alloc_try(size_t bytes, uint64_t *phys) {
     }
     hipSetDevice(S.device);
     void *h = nullptr, *d = nullptr;
-    hipError_t e = hipHostMalloc(&h, bytes, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc(&h, bytes, hipHostMallocCoherent | hipHostMallocMapped);
+    void *hd = nullptr;
+    if (e == hipSuccess) e = hipHostGetDevicePointer(&hd, h, 0);
     if (e == hipSuccess) e = hipMalloc(&d, bytes);
     if (e != hipSuccess) {
         snprintf(S.last_err, sizeof S.last_err, "%zu bytes failed after %.1f MiB already allocated: %s", bytes,
@@ -235,7 +266,7 @@ extern "C" void *fpga_alloc_try(size_t bytes, uint64_t *phys) {
         hipFree(d);
         return nullptr;
     }
-    Buf b = {(uint8_t *)h, (uint8_t *)d, bytes};
+    Buf b = {(uint8_t *)h, (uint8_t *)d, (uint8_t *)hd, bytes};
     S.bufs.insert(std::upper_bound(S.bufs.begin(), S.bufs.end(), b,
                                    [](const Buf &x, const Buf &y) { return x.dev < y.dev; }),
                   b);
@@ -303,6 +334,8 @@ extern "C" void fpga_close(void) {
     S.sstage = nullptr;
     S.ostage = nullptr;
     S.ostage_n = 0;
+    if (S.done) hipHostFree(S.done);
+    S.done = S.done_dev = nullptr;
     if (S.st) hipStreamDestroy(S.st);
     S.st = nullptr;
     S.total = 0;

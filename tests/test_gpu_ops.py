@@ -273,6 +273,33 @@ def test_weights_stay_resident_activations_do_not(drv):
     assert (np.abs(got - ref) <= 1e-5 * mag).all()
 
 
+@pytest.mark.parametrize("n,d,gs", [(288, 288, 32), (64, 1, 64), (4864, 65, 32)])
+def test_every_call_reads_its_activations_and_writes_its_outputs(drv, n, d, gs):
+    """60 calls on the same buffers, activations, scales and outputs inside larger ones at offsets that are aligned,
+    4-byte aligned and neither, new values before each and the outputs cleared: bitwise the oracle's, and the bytes
+    around the outputs untouched"""
+    rng = np.random.default_rng(n + d)
+    wq = rng.integers(-128, 128, size=d * n, dtype=np.int8)
+    ws = rng.uniform(1e-4, 2e-2, size=d * n // gs).astype(np.float32)
+    _, pw = drv.put(wq)
+    _, ps = drv.put(ws)
+    xbuf, px = drv.alloc(n + 64)
+    sbuf, pxs = drv.alloc(n // gs * 4 + 64)
+    out, po = drv.alloc(d * 4 + 64)
+    ref = np.empty(d, np.float32)
+    for k in range(60):
+        ox, os_, oo = (16 * (k % 3), 4 * (k % 4), 4 * (k % 5)) if k % 3 else (k % 7, k % 5, k % 6)
+        xq = rng.integers(-128, 128, size=n, dtype=np.int8)
+        xs = rng.uniform(1e-3, 1e-1, size=n // gs).astype(np.float32)
+        xbuf[ox:ox + n] = xq.view(np.uint8)
+        sbuf[os_:os_ + xs.nbytes] = xs.view(np.uint8)
+        out[:] = 0xA5
+        assert drv.matvec(pw, ps, px + ox, pxs + os_, po + oo, n, d, gs) == 0
+        oracle().or_matvec_runq(ptr(ref), ptr(wq), ptr(ws), ptr(xq), ptr(xs), n, d, gs)
+        assert np.array_equal(out[oo:oo + 4 * d], ref.view(np.uint8)), k
+        assert (out[:oo] == 0xA5).all() and (out[oo + 4 * d:] == 0xA5).all()
+
+
 def test_argument_errors(drv, capfd):
     _, p = drv.alloc(1 << 16)
     assert drv.matvec4(p + 8, p, p, p, p, 32, 1, 4) == -1      # not 64-byte aligned
