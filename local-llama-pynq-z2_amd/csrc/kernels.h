@@ -86,6 +86,7 @@ struct AttnArgs {
     const StepCtrl *ctrl;
     float *sc;              // strict mode, long contexts: scores [n_heads][max_pos]
     int long_ctx;           // 1: the launches for long contexts
+    float *one;             // fast mode, long contexts: the merged output [n_heads][hs], then (0, 1) per head
 };
 
 struct EmbedArgs {

@@ -1097,6 +1097,31 @@ hipError_t launch_attention_strict(const AttnArgs &a, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Merge of a head's slices at long contexts (block = head, a thread per element), what the o projection's prologue does
+// with the same operations in the same order, but once instead of in each of its blocks: there every block reads every
+// head's partials (28 heads x 64 slices of 128 floats, 0.9 MB, at 3000 positions of the 7B shape).  Leaves one slice
+// (max 0, sum 1), whose merge in that prologue is the identity.
+__global__ void __launch_bounds__(128) k_attn_combine(AttnArgs a) {
+    __shared__ float wgt[WAVE];
+    const int h = blockIdx.x, SP = a.splits, hs = a.hs, e = min((int)threadIdx.x, hs - 1), lane = threadIdx.x & (WAVE - 1);
+    int S, chunk;
+    att_slices(a.ctrl->pos, SP, &S, &chunk);
+    const int SW = pow2_at_least(S);
+    const float2 st = ((const float2 *)a.ml)[(size_t)h * SP + min(lane, S - 1)];
+    const float *p = a.acc + (size_t)h * SP * hs + e;
+    float x[WAVE];
+#pragma unroll
+    for (int k = 0; k < WAVE; k++) x[k] = p[(size_t)min(k, S - 1) * hs];
+    if (threadIdx.x < WAVE) merge_weights(st, 0, lane, S, SW, lane < SW ? 1 : 0, wgt);
+    __syncthreads();
+    float acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < WAVE; k++)
+        if (k < S) acc += x[k] * wgt[k];
+    if (threadIdx.x < hs) a.one[(size_t)h * hs + threadIdx.x] = acc;
+    if (threadIdx.x == 0) ((float2 *)(a.one + (size_t)a.n_heads * hs))[h] = make_float2(0.0f, 1.0f);
+}
+
 hipError_t launch_attention(const AttnArgs &a, hipStream_t st) {
     const int kv_mul = a.n_heads / a.n_kv;
     // at most 64 slices: the partial buffers and the o projection's merge (PRO_ATTN) hold that many per head
@@ -1111,12 +1136,13 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t st) {
         const size_t lds = attn_short_lds_floats(kv_mul, a.hs) * 4;
         if (a.hs <= WAVE) hipLaunchKernelGGL(k_attention_short<1>, dim3(a.n_kv * a.splits), dim3(nt), lds, st, a);
         else hipLaunchKernelGGL(k_attention_short<2>, dim3(a.n_kv * a.splits), dim3(nt), lds, st, a);
-        return hipGetLastError();
+    } else {
+        const int threads = 256;
+        if (kv_mul * a.hs > 4 * threads) return hipErrorInvalidValue;
+        const size_t lds = attn_lds_floats(kv_mul, a.hs) * 4;
+        hipLaunchKernelGGL(k_attention, dim3(a.n_kv * a.splits), dim3(threads), lds, st, a);
     }
-    const int threads = 256;
-    if (kv_mul * a.hs > 4 * threads) return hipErrorInvalidValue;
-    const size_t lds = attn_lds_floats(kv_mul, a.hs) * 4;
-    hipLaunchKernelGGL(k_attention, dim3(a.n_kv * a.splits), dim3(threads), lds, st, a);
+    if (a.long_ctx) hipLaunchKernelGGL(k_attn_combine, dim3(a.n_heads), dim3(128), 0, st, a);
     return hipGetLastError();
 }
 

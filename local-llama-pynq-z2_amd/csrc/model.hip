@@ -78,7 +78,8 @@ struct llm_model {
     int32_t *head_ids_d = nullptr;
     std::vector<int32_t> head_ids_h;
     float *kc = nullptr, *vc = nullptr, *x = nullptr, *q = nullptr, *att_ml = nullptr, *att_acc = nullptr;
-    float *att_sc = nullptr; // strict mode: scores [n_heads][ctx]
+    float *att_sc = nullptr;  // strict mode: scores [n_heads][ctx]
+    float *att_one = nullptr; // fast mode, long contexts: merged attention, then (0, 1) per head
     float *logits = nullptr, *hist = nullptr, *part_v = nullptr, *hsc = nullptr;
     int8_t *hq = nullptr;
     int *part_i = nullptr;
@@ -222,8 +223,10 @@ hipError_t launch_sampler(llm_model *m) {
 // Whether the step at `pos` takes the launches for long contexts (both kinds are right at any position).  Strict, from
 // 192 positions (a layer's step, one kernel per head / scores and values apart, us: 7B shape 160 positions 73.1 / 73.0,
 // 256 78.0 / 75.5, 3000 170 / 91; 0.5B shape 160 36.8 / 38.0, 256 39.9 / 39.0, 3000 98 / 52; llama2.c 768 160 34.1 /
-// 34.2, 256 37.1 / 35.1; 288 96 30.8 / 31.3, 160 32.4 / 31.7).
-bool long_step(const llm_model *m, int pos) { return m->strict && pos + 1 >= 192; }
+// 34.2, 256 37.1 / 35.1; 288 96 30.8 / 31.3, 160 32.4 / 31.7).  Fast, from 1024 (slices merged in the o projection /
+// merged before it: 7B shape 700 positions 58.0 / 58.0, 1200 62.1 / 59.2, 3000 66.9 / 61.0; 0.5B shape 700 30.8 / 31.7,
+// 1200 34.9 / 31.9, 3000 38.3 / 32.4; llama2.c 768 1000 32.1 / 32.2).
+bool long_step(const llm_model *m, int pos) { return pos + 1 >= (m->strict ? 192 : 1024); }
 
 // Enqueue one decode step on m->st.  prof != NULL records events around every launch.  Kernel kinds whose
 // bit is set in `skip` are left out (the in-graph timing of llm_profile_graph compares such steps).  With
@@ -314,6 +317,7 @@ int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finaliz
         t.ctrl = m->ctrl;
         t.sc = m->att_sc;
         t.long_ctx = lng;
+        t.one = m->att_one;
         if (on(K_ATTN)) {
             mark(K_ATTN, kind_bytes(m, K_ATTN, pos_hint));
             if (m->strict) {
@@ -331,6 +335,11 @@ int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finaliz
         a.n_heads = I.n_heads;
         a.head_size = m->hs;
         a.att_splits = m->strict ? 1 : m->att_splits; // strict: one slice, merged as the identity
+        if (!m->strict && lng) { // merged already
+            a.att_acc = m->att_one;
+            a.att_ml = m->att_one + dim;
+            a.att_splits = 1;
+        }
         a.out = m->x;
         if (on(K_O)) {
             mark(K_O, kind_bytes(m, K_O, pos_hint));
@@ -544,6 +553,7 @@ int finish_setup(llm_model *m) {
         dalloc(m, &m->att_ml, (size_t)I.n_heads * m->att_splits * 2 * 4) ||
         dalloc(m, &m->att_acc, (size_t)I.n_heads * m->att_splits * m->hs * 4) ||
         dalloc(m, &m->att_sc, (size_t)I.n_heads * m->ctx * 4) ||
+        dalloc(m, &m->att_one, (size_t)(I.dim + 2 * I.n_heads) * 4) ||
         dalloc(m, &m->logits, (size_t)I.n_logits * 4) || dalloc(m, &m->part_v, (size_t)head_grid * 4) ||
         dalloc(m, &m->part_i, (size_t)head_grid * 4) || dalloc(m, &m->hq, (size_t)I.hidden_dim) ||
         dalloc(m, &m->hsc, (size_t)I.hidden_dim / m->gs * 4) || dalloc(m, &m->ctrl, sizeof(StepCtrl)) ||

@@ -347,3 +347,27 @@ def test_host_programs_text_prompts_match_reference(name, tmp_path):
                        input=run.get("stdin", "").encode())
     assert r.returncode == 0, r.stderr.decode(errors="replace")
     assert r.stdout == bytes.fromhex(run["stdout_hex"])
+
+
+@pytest.mark.parametrize("shape", [("dim=512", "heads=4", "kv_heads=2"), ("dim=384", "heads=8", "kv_heads=1"),
+                                   ("dim=128", "heads=8", "kv_heads=4")])
+@pytest.mark.parametrize("ctx", [1100, 4200])
+def test_fast_decode_across_the_long_context_switch(tmp_path, shape, ctx):
+    """fast decode steps at positions 1015 .. 1040 over a prefilled cache, across the switch (1024 positions) to the
+    launches that merge the attention slices before the o projection: the oracle's logits within 2e-2 of their scale
+    at every position (the bar where an int8 step of the layer's later inputs falls the other way) and within 1e-4 at
+    most of them (one layer: its K/V rows come before any attention).  Head sizes 128, 48 and 16; contexts whose
+    slices hold at most 64 positions and more"""
+    p = synth("qwb", str(tmp_path / "f.qwb"), "tiny", 11, *shape, "hidden=256", "layers=1", "vocab=512", "head_k=256",
+              f"max_seq={ctx}")
+    m, om = pkg().Model(p, ctx), OracleModel(p, ctx)
+    ids = [int(om.head_ids[v]) for v in np.random.default_rng(5).integers(2, om.n, 1041)]
+    m.prefill(ids[:1015])
+    err = []
+    for pos, t in enumerate(ids):
+        ref = om.forward(t, pos)
+        if pos >= 1015:
+            err.append(rel_err(m.forward(t, pos), ref))
+    assert max(err) < 2e-2 and np.median(err) < 1e-4, err
+    m.close()
+    om.close()
