@@ -126,7 +126,8 @@ def group_dots(w, xq, n, d, bits, gs=32):
 def prefill_gemm(w, ws, xq, xs, M, n, d, bits, gs=32, rb=16, shape=0):
     """The prefill GEMM (int8 MFMA) on caller data: [M, d] float32.  bits 4/8: qwen planes with fp16 scales;
     bits 0: runq int8 with fp32 scales, group gs.  shape: 0 the library's choice, 10 TA + TB one wave per
-    16 TA rows x 16 TB tokens (TA 1, 2; TB 1, 2, 4), 32 and 33 the 32 x 32 tiles (int4) in the strict and the fast form."""
+    16 TA rows x 16 TB tokens (TA 1, 2; TB 1, 2, 4), 32 and 33 the 32 x 32 tiles (int4) in the strict and the fast form,
+    13 the 16 x 16 tiles (int4) in the fast form."""
     w = np.ascontiguousarray(w).view(np.uint8)
     ws = np.ascontiguousarray(ws)
     xq = np.ascontiguousarray(xq, dtype=np.int8)

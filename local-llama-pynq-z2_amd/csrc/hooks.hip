@@ -91,8 +91,8 @@ extern "C" int mvh_group_dots(const uint8_t *w, const int8_t *xq, int n, int d, 
 
 extern "C" int mvh_prefill_gemm(const uint8_t *w, const void *ws, const int8_t *xq, const float *xs, int M, int n,
                                 int d, int bits, int gs, int rb, int shape, float *y) {
-    const int fast = shape == 33; // k_pgemm32 with the fast mode's sums
-    if (fast) shape = PGEMM_SHAPE_32;
+    const int fast = shape == 33 || shape == 13; // the fast mode's sums: k_pgemm32, k_pgemm's 16 x 16 tiles
+    if (fast) shape = shape == 33 ? PGEMM_SHAPE_32 : 11;
     const int wbits = bits == 0 ? 8 : bits, sf32 = bits == 0;
     if (!w || !ws || !xq || !xs || !y || M < 1 || n <= 0 || d <= 0 || d % 4 || n % 16 ||
         (bits != 0 && bits != 4 && bits != 8) || (gs != 32 && gs != 64) || (bits != 0 && gs != 32) || n % gs ||
@@ -147,7 +147,7 @@ extern "C" int mvh_prefill_gemm(const uint8_t *w, const void *ws, const int8_t *
         g.y = dy;
         g.M = M;
         g.shape = shape;
-        g.strict = !fast;
+        g.fast = fast;
         int dev = 0;
         hipGetDevice(&dev);
         g.simds = 4 * hip_cu_count(dev);

@@ -988,6 +988,7 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
     g.simds = pa.simds;
     g.qflavor = m->qflavor;
     g.strict = m->strict;
+    g.fast = !m->strict;
     g.hq = m->pf_h;
     g.hsc = m->pf_hs;
     // Tile shapes of the four GEMMs, and with them the layout of each one's input.

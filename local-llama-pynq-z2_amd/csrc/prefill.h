@@ -57,6 +57,7 @@ struct PgemmArgs {
                             // (TA 1, 2, 4; TB 1, 2, 4; not 44); PGEMM_SHAPE_32: k_pgemm32 (pgemm32_takes), the
                             // input in the layout of pf_act_off32
     int simds;              // SIMDs of the device (0: 1024)
+    int fast;               // 1: the fast mode's sums (k_pgemm's FMA, k_pgemm32's); 0: the reference's, bitwise
     // swiglu = 1: W is the gate/up matrix (row-blocks of 16: 8 gate rows, then the 8 matching up rows) and the
     // epilogue writes h = silu(gate) * up quantized (groups of 32, flavour qflavor; strict: the reference
     // libm's expf) into the token-block tiles hq / hsc instead of y (int4 weights, shapes 11, 12, 21, 22, PGEMM_SHAPE_32);
@@ -91,12 +92,12 @@ static inline bool pgemm32_takes(const TiledMat &W) {
 }
 // The shape of one of the model's GEMMs.  k_pgemm32 where it has 7/8 of a wave of 32 rows x 32 tokens per SIMD (measured,
 // k_pgemm's tile / k_pgemm32, us: 0.5B shape, 1024 tokens, o and down, 896 waves: 8.2 / 7.8, 28.6 / 26.4; 512 tokens, 448
-// waves: 6.0 / 7.7, 18.0 / 25.9, QKV, 576 waves: 10.6 / 10.4); with the SwiGLU epilogue 2.25 waves of 64 rows x 32
+// waves: 6.0 / 7.7, 18.0 / 25.9, QKV, 576 waves: 10.6 / 10.4); with the SwiGLU epilogue 2 waves of 64 rows x 32
 // tokens (512 tokens of the 0.5B shape, 2432 waves: 30.9 / 28.1, strict 34.0 / 34.4; 77 of the 7B shape, 1776: 62.6 / 71).
 static inline int pgemm_shape(const TiledMat &W, int M, int simds, bool swiglu) {
     if (simds <= 0) simds = 1024;
     const long tiles = (long)((W.rows + 31) / 32) * ((M + 31) / 32);
-    if (pgemm32_takes(W) && (swiglu ? 2 * tiles >= 9L * simds : 8 * tiles >= 7L * simds)) return PGEMM_SHAPE_32;
+    if (pgemm32_takes(W) && (swiglu ? tiles >= 4L * simds : 8 * tiles >= 7L * simds)) return PGEMM_SHAPE_32;
     return pgemm_pick_shape(W.rows, M, simds);
 }
 

@@ -84,8 +84,12 @@ __device__ __forceinline__ void lane_row_transpose(uint32_t (&x)[4]) {
 
 // EK: the epilogue: 0 stores y, 1 SwiGLU + quantization of h (PgemmArgs::swiglu), 2 bias + RoPE + the q / K / V
 // writes (PgemmArgs::qkv)
-template <int WB, int GSZ, int SF32, int TA, int TB, int EK>
+// FMA (the fast mode's 16 x 16 tiles, int4): the product joins the sum unrounded, two instructions per output and group
+// instead of three, and groups 4 q + e go to sum e, the four added at the end: fewer roundings and shorter chains than
+// the reference's order.
+template <int WB, int GSZ, int SF32, int TA, int TB, int EK, int FMA = 0>
 __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
+    static_assert(!FMA || (WB == 4 && TA == 1 && TB == 1), "the fast sums' tiles");
     constexpr bool SWG = EK == 1;
     constexpr int KC = GSZ / 32;             // 32-element chunks per group
     constexpr int AP = WB == 4 ? 1 : 2 * KC; // 16-byte pieces per (row, group) weight segment
@@ -276,13 +280,19 @@ __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
             }
         }
     };
-    float acc[TA][TB][4];
+    float acc[TA][TB][4], part[FMA ? 4 : 1][4]; // FMA: the four sums
 #pragma unroll
     for (int i = 0; i < TA; i++)
 #pragma unroll
         for (int j = 0; j < TB; j++)
 #pragma unroll
             for (int k = 0; k < 4; k++) acc[i][j][k] = 0.0f;
+    if constexpr (FMA) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) part[e][k] = 0.0f;
+    }
     // the weight scales of this lane's output rows for group e of the step in buffer k, read from LDS one
     // group ahead of their use (by group parity)
     float4 scw[2][TA], scn[2][TA];
@@ -307,6 +317,10 @@ __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     float p = SF32 ? (float)d[i][j][r] * wsv[r] : fmaf(__int_as_float(d[i][j][r]), wsv[r], ncv[r]);
+                    if constexpr (FMA) {
+                        part[e][r] = fmaf(p, xe, part[e][r]);
+                        continue;
+                    }
                     p = p * xe; // qwen.c:452, runq.c:452
                     acc[i][j][r] = acc[i][j][r] + p;
                 }
@@ -410,6 +424,10 @@ __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
             for (int ee = 0; ee < 4; ee++)
                 if (kk == k && ee == e) products(d[ee & 1], kk, ee, nullptr);
     }
+    if constexpr (FMA) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[0][0][r] = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
+    }
     if constexpr (EK == 2) {
         // k_p_qkv's operations on the tile (qwen.c:515-524 / runq.c:500-521): lane row k of row tile i holds row
         // R = r0 + 16 i + 4 q + k of token m; its NeoX partner R ^ 8 (same block of 16) is lane row k of the lane
@@ -418,7 +436,7 @@ __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
         const int dim = a.dim, kvd = a.kv_dim, hs = a.head_size, half = hs / 2, rot = dim + kvd;
         const bool neox = a.rope_kind == ROPE_NEOX;
         qkv_operands();
-        float part[TA][TB][4];
+        float prt[TA][TB][4];
 #pragma unroll
         for (int i = 0; i < TA; i++)
 #pragma unroll
@@ -428,7 +446,7 @@ __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
                     // the NeoX partner, from the lane across the halves (every lane takes part in the swap)
                     const uint32_t vb = __float_as_uint(acc[i][j][k]);
                     const auto sw = __builtin_amdgcn_permlane32_swap(vb, vb, false, false);
-                    part[i][j][k] = __uint_as_float((q >> 1) ? sw[0] : sw[1]);
+                    prt[i][j][k] = __uint_as_float((q >> 1) ? sw[0] : sw[1]);
                 }
 #pragma unroll
         for (int i = 0; i < TA; i++)
@@ -448,7 +466,7 @@ __global__ void __launch_bounds__(256) k_pgemm(PgemmArgs a) {
                             const bool first = r < 8;
                             const int e = hh * hs + (first ? ii : half + ii);
                             const float c = pc[i][j][k], sn = ps[i][j][k];
-                            const float self = v + pb[i][j][k], partner = part[i][j][k] + pbp[i][j][k];
+                            const float self = v + pb[i][j][k], partner = prt[i][j][k] + pbp[i][j][k];
                             float o;
                             if (first) { float t1 = self * c, t2 = partner * sn; o = t1 - t2; }
                             else { float t1 = self * c, t2 = partner * sn; o = t1 + t2; }
@@ -830,13 +848,13 @@ hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStre
         const long tiles = (long)((W.rows + br - 1) / br) * ((a.M + 63) / 64);
         const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
         if (a.swiglu) {
-            if (a.strict) hipLaunchKernelGGL((k_pgemm32<1, 0>), grid, dim3(256), 0, st, a);
+            if (!a.fast) hipLaunchKernelGGL((k_pgemm32<1, 0>), grid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_pgemm32<1, 1>), grid, dim3(256), 0, st, a);
         } else if (a.qkv) {
-            if (a.strict) hipLaunchKernelGGL((k_pgemm32<2, 0>), grid, dim3(256), 0, st, a);
+            if (!a.fast) hipLaunchKernelGGL((k_pgemm32<2, 0>), grid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_pgemm32<2, 1>), grid, dim3(256), 0, st, a);
         } else {
-            if (a.strict) hipLaunchKernelGGL((k_pgemm32<0, 0>), grid, dim3(256), 0, st, a);
+            if (!a.fast) hipLaunchKernelGGL((k_pgemm32<0, 0>), grid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_pgemm32<0, 1>), grid, dim3(256), 0, st, a);
         }
         return hipGetLastError();
@@ -852,6 +870,10 @@ hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStre
             return hipErrorInvalidValue;
         const int xt = (W.rows + 16 * TA - 1) / (16 * TA), yt = (a.M + 16 * TB - 1) / (16 * TB);
         const unsigned blocks = (unsigned)(8 * ((xt + 7) / 8) * ((yt + 3) / 4));
+        if (wbits == 4 && TA == 1 && a.fast) {
+            hipLaunchKernelGGL((k_pgemm<4, 32, 0, 1, 1, 2, 1>), dim3(blocks), dim3(256), 0, st, a);
+            return hipGetLastError();
+        }
 #define PGQ(WB_, GS_, SF_, T_)                                                                                 \
         if (wbits == WB_ && gs == GS_ && sf32 == SF_ && TA == T_) {                                           \
             hipLaunchKernelGGL((k_pgemm<WB_, GS_, SF_, T_, T_, 2>), dim3(blocks), dim3(256), 0, st, a);       \
@@ -870,6 +892,10 @@ hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStre
         const int RT = 4 / TA, NTY = 4 / RT;
         const int xt = W.rows / (16 * TA), yt = (a.M + 16 * TB - 1) / (16 * TB);
         const unsigned blocks = (unsigned)(8 * ((xt / RT + 7) / 8) * ((yt + NTY - 1) / NTY));
+        if (TA == 1 && TB == 1 && a.fast) {
+            hipLaunchKernelGGL((k_pgemm<4, 32, 0, 1, 1, 1, 1>), dim3(blocks), dim3(256), 0, st, a);
+            return hipGetLastError();
+        }
 #define PGS(TA_, TB_)                                                                                          \
         if (TA == TA_ && TB == TB_) {                                                                         \
             hipLaunchKernelGGL((k_pgemm<4, 32, 0, TA_, TB_, 1>), dim3(blocks), dim3(256), 0, st, a);         \
@@ -878,6 +904,12 @@ hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStre
         PGS(1, 1) PGS(1, 2) PGS(2, 1) PGS(2, 2)
 #undef PGS
         return hipErrorInvalidValue;
+    }
+    if (a.fast && wbits == 4 && shape == 11) {
+        const int xt = (W.rows + 15) / 16, yt = (a.M + 15) / 16;
+        const unsigned blocks = (unsigned)(8 * ((xt + 7) / 8) * ((yt + 3) / 4));
+        hipLaunchKernelGGL((k_pgemm<4, 32, 0, 1, 1, 0, 1>), dim3(blocks), dim3(256), 0, st, a);
+        return hipGetLastError();
     }
 #define PGW(WB_, GS_, SF_, TA_, TB_)                                                                           \
     if (TA == TA_ && TB == TB_) {                                                                             \

@@ -74,7 +74,7 @@ def test_prefill_gemm_bit_exact_special_scales(bits, shape):
 @pytest.mark.parametrize("M,n,d,rb", [(1, 64, 36, 16), (33, 128, 100, 8), (64, 896, 64, 16), (95, 4864, 160, 8),
                                       (31, 192, 32, 32), (600, 256, 1152, 16)])
 def test_prefill_gemm32_exact_and_fast(M, n, d, rb):
-    """the 32 x 32 tiles: rows and tokens that fill no tile, one, or end inside one,
+    """the 32 x 32 tiles (and the 16 x 16 ones in the fast form): rows and tokens that fill no tile, one, or end inside one,
     1 to 76 steps of two groups, records of 2 to 8 groups, special scales in the first rows: bitwise the oracle's in
     the strict form; the fast form leaves the last product of a term unrounded, so it is held to n/32 roundings of
     2^-24 of the sum of the terms' magnitudes against float64"""
@@ -86,12 +86,13 @@ def test_prefill_gemm32_exact_and_fast(M, n, d, rb):
     xq[0] = -128
     xs = rng.uniform(1e-3, 1e-1, size=(M, n // 32)).astype(np.float32)
     check_qwen_gemm(w, s, xq, xs, M, n, d, 4, rb, 32)
-    y = pkg().prefill_gemm(w, s, xq, xs, M, n, d, 4, 32, rb, 33)
+    fast = [pkg().prefill_gemm(w, s, xq, xs, M, n, d, 4, 32, rb, shape) for shape in (33, 13)]
     wv = unpack_q4(w, d, n).reshape(d, -1, 32).astype(np.float64) * s.view(np.float16).reshape(d, -1, 1).astype(np.float64)
     xv = xq.reshape(M, -1, 32).astype(np.float64) * xs[..., None].astype(np.float64)
     terms = np.einsum("dgk,mgk->mdg", wv, xv)
-    err, size = np.abs(y - terms.sum(2)), np.abs(terms).sum(2)
-    assert (err <= (n // 32 + 1) * 2.0 ** -24 * size).all()
+    for y in fast:
+        err, size = np.abs(y - terms.sum(2)), np.abs(terms).sum(2)
+        assert (err <= (n // 32 + 1) * 2.0 ** -24 * size).all()
 
 
 @pytest.mark.parametrize("shape", SHAPES)
