@@ -108,7 +108,8 @@ int llm_profile_graph(llm_model *m, int steps, int rounds, llm_kernel_stat *stat
  * position n-1.  Returns 0 or -1. */
 int llm_prefill(llm_model *m, const int *ids, int n, float *logits);
 /* Whether llm_generate runs the prompt through llm_prefill (on by default) or one decode step per prompt
- * position.  The --logits history (llm_generate with `logits`) always uses the per-position steps. */
+ * position.  A generation that keeps every position's
+ * logits takes the prompt through it too, the head as one GEMM (where its row count is a multiple of 4). */
 int llm_set_prefill(llm_model *m, int on);
 
 /* Reference-order ("strict") mode on or off; no counterpart in the reference, whose CPU loops are this order

@@ -349,3 +349,39 @@ def test_strict_prefill_attention_equals_the_per_position_path(tmp_path, fmt, sh
         ref = om.forward(t, pos)
     assert np.array_equal(lg, ref)
     om.close()
+
+
+@pytest.mark.parametrize("fmt,shape,n,strict,temp", [("qwb", ("dim=256", "heads=4", "kv_heads=2"), 37, True, 0.0),
+                                                     ("qwb", ("dim=256", "heads=4", "kv_heads=2"), 2060, True, 0.0),
+                                                     ("qwb", ("dim=384", "heads=4", "kv_heads=2"), 150, True, 0.8),
+                                                     ("bin", ("dim=256", "heads=4", "kv_heads=4", "gs=64"), 90, True, 0.8),
+                                                     ("bin", ("dim=256", "heads=4", "kv_heads=4"), 65, False, 0.0),
+                                                     ("qwb", ("dim=256", "heads=4", "kv_heads=2"), 65, False, 0.0),
+                                                     ("qwb254", ("dim=256", "heads=4", "kv_heads=2"), 30, True, 0.0)])
+def test_logits_history_through_the_batched_prompt(tmp_path, fmt, shape, n, strict, temp):
+    """llm_generate with every position's logits: the prompt in one batched pass (the head as a GEMM) against the steps
+    one by one.  Strict: logits, ids and the sampler's draws bit for bit, one chunk and two (2060 tokens), fp16 and
+    fp32 scales, groups of 64; a head of 254 rows, which the GEMM does not take, keeps the steps.  Fast: each
+    position's logits within 2e-2 of their scale (the flip-limited bar) and within 1e-3 at most of them"""
+    ctx = n + 30
+    extra = ["hidden=256", "layers=1" if not strict else "layers=2", "vocab=512", f"max_seq={ctx}"]
+    extra += ["head_k=254" if fmt == "qwb254" else "head_k=256"] if fmt != "bin" else []
+    p = synth(fmt[:3], str(tmp_path / f"g.{fmt[:3]}"), "tiny", 13, *shape, *extra)
+    runs = []
+    for on in (False, True):
+        m = pkg().Model(p, ctx)
+        hid = m.head_ids if fmt != "bin" else np.arange(512)
+        ids = [int(hid[v]) for v in np.random.default_rng(n).integers(2, len(hid), n)]
+        m.set_strict(strict)
+        m.set_prefill(on)
+        if temp:
+            m.set_sampler(temp, 0.9, 77)
+        r = m.generate(ids, 9, logits=True)
+        runs.append((r["ids"], r["logits"]))
+        m.close()
+    (ids_a, lg_a), (ids_b, lg_b) = runs
+    if strict:
+        assert np.array_equal(ids_a, ids_b) and np.array_equal(lg_a, lg_b)
+    else:
+        err = [rel_err(y, x) for x, y in zip(lg_a[:n], lg_b[:n])]
+        assert max(err) < 2e-2 and np.median(err) < 1e-3, err
