@@ -1521,23 +1521,27 @@ __global__ void __launch_bounds__(256) k_p_attn_strict(ProwArgs a) {
 //   softmax: the row's maximum, expf (ref_expf) per position, and the sum in position order: the tile's exponentials
 //     go through a small LDS tile of the wave, lane r adds row r;
 //   values: lane = element (two per lane for a head size of 128).  The probabilities e / sum of a tile go through
-//     the same LDS tile into the DPP layout, V rows come straight from memory, 16 positions in flight ahead.
+//     the same LDS tile into the DPP layout; V tiles come through the K tile's place in LDS (read straight from memory
+//     by each wave, a load per 4 to 8 vector instructions kept the CU's load path busy: 2011 tokens of the 0.5B shape
+//     in one launch 283 -> 262 us).
 // The floor is the 4 VALU instructions per row, position and 64 elements (multiply and add are rounded separately,
 // so there is no FMA and no MFMA in it).  Positions past a row's own token take no part (they are selected away, so
 // nothing that a later token holds can reach the row).
 //
 // More rows per wave share its loads and overheads, fewer give more waves (the launcher's rule).  Measured, per layer:
 // 512 tokens of the Qwen2-0.5B shape 51.6 us with a tile of rows per block and LDS-fed chains, now 40; 2011 tokens in
-// one launch 283-308 us for 184 us of multiplies and adds (39.3 T lane operations/s), 980 us before.
+// one launch 262 us for 184 us of multiplies and adds (39.3 T lane operations/s), 980 us before.  Score rows in LDS
+// where they fit measured the same, and so did rounds of blocks in alternating order.
 #define SPW_T 64
 __host__ __device__ inline int spw_rows_pad(int M, int kv_mul) { return (M * kv_mul + 15) / 16 * 16; }
 template <int HS, int R>
 __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) {
     constexpr int KP = HS + 4, NQ = HS / 16, VE = HS > 64 ? 2 : 1, FV = HS * SPW_T / 1024;
     static_assert(HS % 16 == 0 && (HS <= 64 || HS == 128), "head sizes of the row kernel");
-    __shared__ __align__(16) float kt[SPW_T * KP];
-    __shared__ __align__(16) float et[4][R][SPW_T + 4];
+    __shared__ __align__(16) float kt[SPW_T * KP];            // a K or V tile
+    __shared__ __align__(16) float ets[4][R][SPW_T + 4];
     const int tid = threadIdx.x, l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = l & 15;
+    float(*et)[SPW_T + 4] = ets[w];                           // this wave's tile of exponentials or probabilities
     const int kvh = blockIdx.x, kv_mul = a.n_heads / a.n_kv, rows = a.M * kv_mul;
     // the longest causal ranges first
     const int b0 = 4 * R * ((int)gridDim.y - 1 - (int)blockIdx.y), row0 = b0 + w * R;
@@ -1554,7 +1558,7 @@ __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) 
     // (a position past the block's last reads zeros through an out-of-range offset)
     const auto rs_k = __builtin_amdgcn_make_buffer_rsrc((void *)(a.kc + koff), 0, nrec, PG_RSRC3);
     const auto rs_v = __builtin_amdgcn_make_buffer_rsrc((void *)(a.vc + koff), 0, nrec, PG_RSRC3);
-    float *scr[R];
+    float *scr[R]; // lane l's score of position t0 + l of row r: scr[r][t0]
 #pragma unroll
     for (int r = 0; r < R; r++)
         scr[r] = a.att_sc + ((size_t)kvh * spw_rows_pad(a.M, kv_mul) + row0 + r) * SP + l;
@@ -1564,36 +1568,42 @@ __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) 
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
+    // a K or V tile: all of a thread's loads in flight at once, then its stores
+    float4 f[FV];
+    auto fetch = [&](__amdgpu_buffer_rsrc_t rs, int t0) {
+#pragma unroll
+        for (int j = 0; j < FV; j++) {
+            const int idx = tid + 256 * j, tt = idx / (HS / 4), c = idx - tt * (HS / 4);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+                rs, t0 + tt < Pb ? (uint32_t)((t0 + tt) * a.kv_dim + 4 * c) * 4u : 0x80000000u, 0, 0);
+            f[j] = *(const float4 *)&v;
+        }
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int j = 0; j < FV; j++) {
+            const int idx = tid + 256 * j, tt = idx / (HS / 4), c = idx - tt * (HS / 4);
+            *(float4 *)(kt + tt * KP + 4 * c) = f[j];
+        }
+    };
     float mx[R];
     {
+        fetch(rs_k, 0);
         float qv[R][NQ];
 #pragma unroll
         for (int r = 0; r < R; r++)
 #pragma unroll
             for (int c = 0; c < NQ; c++) qv[r][c] = a.q[(size_t)tok[r] * a.dim + head[r] * HS + 16 * c + l16];
-        float4 f[FV];
-        auto fetch = [&](int t0) {
-#pragma unroll
-            for (int j = 0; j < FV; j++) {
-                const int idx = tid + 256 * j, tt = idx / (HS / 4), c = idx - tt * (HS / 4);
-                const auto v = __builtin_amdgcn_raw_buffer_load_b128(
-                    rs_k, t0 + tt < Pb ? (uint32_t)((t0 + tt) * a.kv_dim + 4 * c) * 4u : 0x80000000u, 0, 0);
-                f[j] = *(const float4 *)&v;
-            }
-        };
         const float rs = sqrtf((float)HS);
 #pragma unroll
         for (int r = 0; r < R; r++) mx[r] = -INFINITY;
-        fetch(0);
         for (int t0 = 0; t0 < Pb; t0 += SPW_T) {
             __syncthreads(); // the previous tile is consumed
-#pragma unroll
-            for (int j = 0; j < FV; j++) {
-                const int idx = tid + 256 * j, tt = idx / (HS / 4), c = idx - tt * (HS / 4);
-                *(float4 *)(kt + tt * KP + 4 * c) = f[j];
-            }
+            put();
             __syncthreads();
-            fetch(t0 + SPW_T);
+            if (t0 + SPW_T < Pb) fetch(rs_k, t0 + SPW_T);
+            else fetch(rs_v, 0); // the first V tile, in flight during the softmax
+            if (t0 >= Pw) continue;
             const float *kr = kt + l * KP;
             float d[R];
 #pragma unroll
@@ -1621,7 +1631,6 @@ __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) 
             }
         }
     }
-    if (row0 >= rows) return; // the whole wave (no barrier below)
 
     float sum[R];
     {
@@ -1642,10 +1651,10 @@ __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) 
             for (int r = 0; r < R; r++) {
                 e[r] = t0 + l < P[r] ? ref_expf(e[r] - mx[r]) : 0.0f; // (+0 leaves the sum, never -0, unchanged)
                 scr[r][t0] = e[r];
-                et[w][r][l] = e[r];
+                et[r][l] = e[r];
             }
             wave_sync();
-            const float4 *er = (const float4 *)et[w][l & (R - 1)];
+            const float4 *er = (const float4 *)et[l & (R - 1)];
             float4 x[SPW_T / 4];
 #pragma unroll
             for (int j = 0; j < SPW_T / 4; j++) x[j] = er[j];
@@ -1666,53 +1675,47 @@ __global__ void __launch_bounds__(256) k_p_attn_strict_rows(ProwArgs a, int SP) 
 #pragma unroll
     for (int k = 0; k < R * VE; k++) acc[k] = 0.0f;
     {
-        const uint32_t vo = (HS >= 64 || l < HS ? l : 0) * 4 * VE;
-        const int vstep = a.kv_dim * 4;
-        float v[2][16][VE];
-        auto vload = [&](int k, int t0) { // V of positions t0 .. t0 + 15
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int so = min(t0 + i, Pb - 1) * vstep; // (past the last position: its row, selected away)
-                if constexpr (VE == 1) {
-                    v[k][i][0] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_v, vo, so, 0));
-                } else {
-                    const auto x = __builtin_amdgcn_raw_buffer_load_b64(rs_v, vo, so, 0);
-                    v[k][i][0] = __int_as_float(x[0]);
-                    v[k][i][1] = __int_as_float(x[1]);
-                }
-            }
-        };
+        const float *vl = kt + (HS >= 64 || l < HS ? l : 0) * VE;
         float nx[R];
 #pragma unroll
         for (int r = 0; r < R; r++) nx[r] = scr[r][0];
-        vload(0, 0);
         const int Pmin = P[0];
-        for (int t0 = 0; t0 < Pw; t0 += SPW_T) {
+        for (int t0 = 0; t0 < Pb; t0 += SPW_T) {
+            __syncthreads(); // the previous tile is consumed
+            put();
+            __syncthreads();
+            fetch(rs_v, t0 + SPW_T); // (past the last tile: zeros, no traffic)
+            if (t0 >= Pw) continue;
 #pragma unroll
-            for (int r = 0; r < R; r++) et[w][r][l] = nx[r] / sum[r];
+            for (int r = 0; r < R; r++) et[r][l] = nx[r] / sum[r];
             wave_sync();
             const int tn = t0 + SPW_T < Pw ? t0 + SPW_T : t0;
 #pragma unroll
             for (int r = 0; r < R; r++) nx[r] = scr[r][tn];
-            float pr[R][4];
-#pragma unroll
-            for (int r = 0; r < R; r++)
-#pragma unroll
-                for (int c = 0; c < 4; c++) pr[r][c] = et[w][r][16 * c + l16];
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const int tc = t0 + 16 * c;
-                vload((c + 1) & 1, tc + 16);
-                float pc[R];
+                float pc[R], v[16][VE];
 #pragma unroll
-                for (int r = 0; r < R; r++) pc[r] = pr[r][c];
-                if (tc + 16 <= Pmin) chain16<R * VE, VE>(acc, pc, v[c & 1], [](int, int) { return true; });
+                for (int r = 0; r < R; r++) pc[r] = et[r][16 * c + l16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    if constexpr (VE == 1) {
+                        v[i][0] = vl[(16 * c + i) * KP];
+                    } else {
+                        const float2 x = *(const float2 *)(vl + (16 * c + i) * KP);
+                        v[i][0] = x.x;
+                        v[i][1] = x.y;
+                    }
+                }
+                if (tc + 16 <= Pmin) chain16<R * VE, VE>(acc, pc, v, [](int, int) { return true; });
                 else // positions that some row of the wave does not see
-                    chain16<R * VE, VE>(acc, pc, v[c & 1], [&](int i, int k) { return tc + i < P[k / VE]; });
+                    chain16<R * VE, VE>(acc, pc, v, [&](int i, int k) { return tc + i < P[k / VE]; });
             }
             wave_sync();
         }
     }
+    if (row0 >= rows) return; // the whole wave (no barrier below)
     if (HS % a.gs) { // quantization groups that cross heads: k_p_quant_rows quantizes the rows afterwards
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -1792,18 +1795,18 @@ hipError_t launch_p_attention(const ProwArgs &a, hipStream_t st) {
         if (prefill_strict_rows(hs)) {
             const int kvm = a.n_heads / a.n_kv, rows = a.M * kvm, SP = prefill_strict_sp(a.p0 + a.M);
             if (!a.att_sc) return hipErrorInvalidValue;
-            // rows per wave: 4 from 9 rows per SIMD, 2 from 3.5, else 1 (whole strict prefills of two layers, 1024 SIMDs,
-            // R = 4 / 2 / 1, us: Qwen2-0.5B shape 200 tokens, 2800 rows: 248 / 234 / 231; 300: 281 / 261 / 269; 512:
-            // 317 / 309 / 331; 1024, 14336 rows: 503 / 524 / 628; 7B shape 300, 8400 rows: 1034 / 1034 / 1072; 512:
-            // 1453 / 1473 / 1586)
+            // rows per wave: 4 from 14 rows per SIMD, 2 from 5.5, else 1 (whole strict prefills of two layers, 1024 SIMDs,
+            // R = 4 / 2 / 1, us: Qwen2-0.5B shape 200 tokens, 2800 rows: 245 / 231 / 222; 512, 7168 rows: 328 / 306 / 320;
+            // 1024, 14336 rows: 490 / 473 / 524; 2011: 943 / 990 / 1204; 7B shape 200, 5600 rows: 800 / 778 / 782; 512,
+            // 14336 rows: 1363 / 1368 / 1414; 700: 1749 / 1782 / 1877)
             const long all = (long)rows * a.n_kv, simds = a.simds > 0 ? a.simds : 1024;
-            const int R = all >= 9 * simds ? 4 : 2 * all >= 7 * simds ? 2 : 1;
+            const int R = all >= 14 * simds ? 4 : 2 * all >= 11 * simds ? 2 : 1;
             const dim3 grid(a.n_kv, (rows + 4 * R - 1) / (4 * R));
 #define SPW_LAUNCH(H)                                                                                          \
             if (hs == H) {                                                                                     \
-                if (R == 4) hipLaunchKernelGGL((k_p_attn_strict_rows<H, 4>), grid, dim3(256), 0, st, a, SP);   \
+                if (R == 4) hipLaunchKernelGGL((k_p_attn_strict_rows<H, 4>), grid, dim3(256), 0, st, a, SP); \
                 else if (R == 2) hipLaunchKernelGGL((k_p_attn_strict_rows<H, 2>), grid, dim3(256), 0, st, a, SP); \
-                else hipLaunchKernelGGL((k_p_attn_strict_rows<H, 1>), grid, dim3(256), 0, st, a, SP);          \
+                else hipLaunchKernelGGL((k_p_attn_strict_rows<H, 1>), grid, dim3(256), 0, st, a, SP);   \
             }
             SPW_LAUNCH(16) SPW_LAUNCH(32) SPW_LAUNCH(48) SPW_LAUNCH(64) SPW_LAUNCH(128)
 #undef SPW_LAUNCH
