@@ -942,15 +942,33 @@ hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStre
 // ------------------------------------------------------------------------------------------------------
 // per-token element-wise steps (one block of 256 threads per token)
 
+// Threads of a per-token block: rows of up to 4 elements per thread are loaded in one round (the kernels' first NQ or
+// MP passes); longer rows run pass after pass, a round trip each, at 256 threads.  With more tokens than fill the chip
+// the rounds overlap and the smaller blocks win.  256 / 1024 threads at the 7B shape's 3584 elements, us: 77 tokens,
+// embedding 13.8 / 5.2, norm 11.0 / 5.1, slice merge 15.6 / 7.8; 2000 tokens, norm 24.5 / 29.7 (strict 48.2 / 41.9: its
+// sequential sum gets more segments), slice merge 62 / 80.
+static inline int row_threads(int dim, int M, bool strict_norm = false) {
+    return dim <= 1024 || (M > 1024 && !strict_norm) ? 256 : dim <= 2048 ? 512 : 1024;
+}
+
 // embedding rows (qwen.c:498-501, runq.c:490-492)
-__global__ void __launch_bounds__(256) k_p_embed(ProwArgs a) {
-    const int m = blockIdx.x, token = a.ids[m], ngr = a.dim / a.gs;
+__global__ void __launch_bounds__(1024) k_p_embed(ProwArgs a) {
+    const int m = blockIdx.x, token = a.ids[m], ngr = a.dim / a.gs, nt = blockDim.x;
     const int8_t *er = a.emb_q + (size_t)token * a.dim;
-    for (int i = threadIdx.x; i < a.dim; i += blockDim.x) {
-        const int g = i / a.gs;
-        const float sc = a.emb_sf32 ? ((const float *)a.emb_s)[(size_t)token * ngr + g]
-                                    : f16_bits_to_f32(((const uint16_t *)a.emb_s)[(size_t)token * ngr + g]);
-        a.x[(size_t)m * a.dim + i] = (float)er[i] * sc;
+    constexpr int NQ = 4;
+    for (int i0 = threadIdx.x; i0 < a.dim; i0 += NQ * nt) {
+        int8_t q[NQ];
+        float sc[NQ];
+#pragma unroll
+        for (int k = 0; k < NQ; k++) {
+            const int i = min(i0 + k * nt, a.dim - 1), g = i / a.gs;
+            q[k] = er[i];
+            sc[k] = a.emb_sf32 ? ((const float *)a.emb_s)[(size_t)token * ngr + g]
+                               : f16_bits_to_f32(((const uint16_t *)a.emb_s)[(size_t)token * ngr + g]);
+        }
+#pragma unroll
+        for (int k = 0; k < NQ; k++)
+            if (i0 + k * nt < a.dim) a.x[(size_t)m * a.dim + i0 + k * nt] = (float)q[k] * sc[k];
     }
 }
 
@@ -958,8 +976,8 @@ __global__ void __launch_bounds__(256) k_p_embed(ProwArgs a) {
 // With RESID the residual add of the previous GEMM comes first: x[m] += y[m] (qwen.c:551, 565; runq.c:575-577,
 // 603-605), stored back, then normalized.
 template <bool RESID>
-__global__ void __launch_bounds__(256) k_p_norm_quant(ProwArgs a) {
-    extern __shared__ __align__(16) float sv[]; // dim floats + 8, then the strict mode's squares and sum scratch
+__global__ void __launch_bounds__(1024) k_p_norm_quant(ProwArgs a) {
+    extern __shared__ __align__(16) float sv[]; // dim floats + 16, then the strict mode's squares and sum scratch
     const int m = blockIdx.x, n = a.dim, nt = blockDim.x;
     float *x = a.x + (size_t)m * n;
     const float *y = a.y + (size_t)m * n;
@@ -999,7 +1017,7 @@ __global__ void __launch_bounds__(256) k_p_norm_quant(ProwArgs a) {
     }
     float ss;
     if (a.strict) { // one running sum of the rounded squares in element order (qwen.c:339, runq.c:396-398)
-        float *sq = sv + n + 8; // the squares (each rounded, as the reference's), then the sum's scratch
+        float *sq = sv + n + 16; // the squares (each rounded, as the reference's), then the sum's scratch
         __syncthreads();
         for (int i = threadIdx.x; i < n; i += nt) sq[i] = sv[i] * sv[i];
         __syncthreads();
@@ -1424,7 +1442,7 @@ __global__ void __launch_bounds__(256) k_p_attention(ProwArgs a) {
 // merge of token m's S slices: with mx the largest slice max, w_s = exp(max_s - mx) / sum_k l_k exp(max_k - mx)
 // and out[h*hs + e] = sum_s acc_s[e] * w_s, then the row quantized to int8 for the o projection (qwen.c:549,
 // runq.c:571).  Tokens with one slice were done by k_p_flash, unless `all` (then every token is merged here).
-__global__ void __launch_bounds__(256) k_p_attn_merge(ProwArgs a, int all) {
+__global__ void __launch_bounds__(1024) k_p_attn_merge(ProwArgs a, int all) {
     extern __shared__ __align__(16) float sm[]; // dim floats of the row, then [n_heads][att_smax] weights
     float *row = sm, *wgt = sm + a.dim;
     const int m = blockIdx.x, hs = a.head_size, S = (a.p0 + m) / a.att_sl + 1;
@@ -1757,15 +1775,16 @@ __global__ void __launch_bounds__(256) k_p_quant_rows(ProwArgs a) {
 }
 
 hipError_t launch_p_embed(const ProwArgs &a, hipStream_t st) {
-    hipLaunchKernelGGL(k_p_embed, dim3(a.M), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_p_embed, dim3(a.M), dim3(row_threads(a.dim, a.M)), 0, st, a);
     return hipGetLastError();
 }
 hipError_t launch_p_norm_quant(const ProwArgs &a, bool resid, hipStream_t st) {
     if (a.dim % 4 || ((uintptr_t)a.oq & 3)) return hipErrorInvalidValue;
-    // dim floats, 8 for the block sum, then the strict mode's squares and sequential sum's scratch
-    const size_t lds = (size_t)(a.dim + 8) * 4 + (a.strict ? (size_t)a.dim * 4 + seq_sum_scratch_bytes(256) : 0);
-    if (resid) hipLaunchKernelGGL(k_p_norm_quant<true>, dim3(a.M), dim3(256), lds, st, a);
-    else hipLaunchKernelGGL(k_p_norm_quant<false>, dim3(a.M), dim3(256), lds, st, a);
+    // dim floats, a float per wave for the block sum, then the strict mode's squares and sequential sum's scratch
+    const int nt = row_threads(a.dim, a.M, a.strict);
+    const size_t lds = (size_t)(a.dim + 16) * 4 + (a.strict ? (size_t)a.dim * 4 + seq_sum_scratch_bytes(nt) : 0);
+    if (resid) hipLaunchKernelGGL(k_p_norm_quant<true>, dim3(a.M), dim3(nt), lds, st, a);
+    else hipLaunchKernelGGL(k_p_norm_quant<false>, dim3(a.M), dim3(nt), lds, st, a);
     return hipGetLastError();
 }
 hipError_t launch_p_qkv(const ProwArgs &a, hipStream_t st) {
@@ -1842,6 +1861,6 @@ hipError_t launch_p_attention(const ProwArgs &a, hipStream_t st) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if ((a.p0 + a.M - 1) / a.att_sl == 0 && direct) return hipSuccess; // every token has one slice
-    hipLaunchKernelGGL(k_p_attn_merge, dim3(a.M), dim3(256), merge_lds, st, a, direct ? 0 : 1);
+    hipLaunchKernelGGL(k_p_attn_merge, dim3(a.M), dim3(row_threads(a.dim, a.M)), merge_lds, st, a, direct ? 0 : 1);
     return hipGetLastError();
 }
