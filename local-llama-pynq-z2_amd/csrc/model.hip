@@ -1249,6 +1249,14 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
             return -1;
         }
     }
+    const int end_prompt = pos0 + n_prompt; // positions below take their token from the prompt
+    // positions: the prompt, then one per generated token, within the context
+    const int last_pos = std::min(end_prompt - 1 + max_new - 1, m->ctx - 1);
+    const bool batched = m->prefill_on && n_prompt > 1 && (!hist || head_gemm_ok(m));
+    // the captured steps this run launches (both kinds where it crosses their border), before any work is queued
+    const int first_step = batched ? end_prompt : pos0;
+    if (first_step <= last_pos && (!step_graph(m, hist, smp, first_step) || !step_graph(m, hist, smp, last_pos)))
+        return -1;
     auto launch = [&](int pos) -> int {
         hipGraphExec_t g = step_graph(m, hist, smp, pos);
         if (!g) return -1;
@@ -1256,12 +1264,9 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
         return 0;
     };
     HIP_OR_FAIL("llm_generate", hipMemcpy(m->prompt + pos0, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice));
-    const int end_prompt = pos0 + n_prompt; // positions below take their token from the prompt
     if (set_ctrl(m, pos0 - 1, 0, end_prompt, 1)) return -1;
-    // positions: the prompt, then one per generated token, within the context
-    const int last_pos = std::min(end_prompt - 1 + max_new - 1, m->ctx - 1);
     const double t0 = now_ms();
-    if (m->prefill_on && n_prompt > 1 && (!hist || head_gemm_ok(m))) {
+    if (batched) {
         // the prompt in one batched pass; the first decode step then finishes its last position's argmax
         if (prefill_all(m, prompt, n_prompt, smp, pos0, hist)) return -1;
         if (set_ctrl(m, end_prompt - 1, prompt[n_prompt - 1], end_prompt, 1)) return -1;
