@@ -1547,7 +1547,7 @@ __global__ void __launch_bounds__(256) k_p_attn_strict(ProwArgs a) {
 // nothing that a later token holds can reach the row).
 //
 // More rows per wave share its loads and overheads, fewer give more waves (the launcher's rule).  Measured, per layer:
-// 512 tokens of the Qwen2-0.5B shape 51.6 us with a tile of rows per block and LDS-fed chains, now 40; 2011 tokens in
+// 512 tokens of the Qwen2-0.5B shape 51.6 us with a tile of rows per block and LDS-fed chains, now 32; 2011 tokens in
 // one launch 262 us for 184 us of multiplies and adds (39.3 T lane operations/s), 980 us before.  Score rows in LDS
 // where they fit measured the same, and so did rounds of blocks in alternating order.
 #define SPW_T 64
