@@ -901,10 +901,12 @@ int prefill_alloc(llm_model *m, int M) {
     if (M <= m->pf_cap) return 0;
     const llm_info &I = m->info;
     const int dim = I.dim, hid = I.hidden_dim, rows = std::max(dim + 2 * m->kv_dim, 2 * hid), wmax = std::max(dim, hid);
-    for (void *p : {(void *)m->pf_x, (void *)m->pf_y, (void *)m->pf_q, (void *)m->pf_s,
-                    (void *)m->pf_a, (void *)m->pf_ids, (void *)m->pf_ml, (void *)m->pf_acc, (void *)m->pf_h,
-                    (void *)m->pf_hs})
+    auto drop = [](auto *&p) {
         if (p) hipFree(p);
+        p = nullptr;
+    };
+    drop(m->pf_x), drop(m->pf_y), drop(m->pf_q), drop(m->pf_s), drop(m->pf_a), drop(m->pf_ids), drop(m->pf_ml);
+    drop(m->pf_acc), drop(m->pf_h), drop(m->pf_hs);
     m->pf_cap = 0;
     // the GEMM input in token-block tiles (rounded up to 16 tokens, whole chunk pairs and scale quads)
     if (hipMalloc(&m->pf_x, (size_t)M * dim * 4) != hipSuccess || hipMalloc(&m->pf_y, (size_t)M * rows * 4) != hipSuccess ||
@@ -915,7 +917,7 @@ int prefill_alloc(llm_model *m, int M) {
         hipMalloc(&m->pf_acc, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * m->hs * 4) != hipSuccess ||
         hipMalloc(&m->pf_h, pf_act_bytes(hid, M)) != hipSuccess ||
         hipMalloc(&m->pf_hs, pf_scale_floats(hid / m->gs, M) * 4) != hipSuccess) {
-        fprintf(stderr, "llm_prefill: cannot allocate the activations of %d tokens\n", M);
+        hipGetLastError();
         return -1;
     }
     m->pf_cap = M;
@@ -932,7 +934,7 @@ int prefill_alloc_strict(llm_model *m, int M, int end) {
     m->pf_sc = nullptr;
     m->pf_sc_n = 0;
     if (hipMalloc(&m->pf_sc, need * 4) != hipSuccess) {
-        fprintf(stderr, "llm_prefill: cannot allocate the score rows of %d tokens up to position %d\n", M, end);
+        hipGetLastError();
         return -1;
     }
     m->pf_sc_n = need;
@@ -1106,10 +1108,21 @@ int prefill_logits(llm_model *m, int p0, int M) {
 // partials, and (finalize) its argmax into gen[pos0 + n - 1].  Afterwards the step state is position
 // pos0 + n - 1, as after those forward() calls.
 int prefill_all(llm_model *m, const int *ids, int n, bool sampled = false, int pos0 = 0, bool hist = false) {
-    const int chunk = std::min(n, PREFILL_CHUNK);
-    if (prefill_alloc(m, chunk) || prefill_alloc_strict(m, chunk, pos0 + n)) return -1;
-    for (int i = 0; i < n; i += PREFILL_CHUNK) {
-        const int M = std::min(PREFILL_CHUNK, n - i);
+    int chunk = std::min(n, PREFILL_CHUNK);
+    while (prefill_alloc(m, chunk) || prefill_alloc_strict(m, chunk, pos0 + n)) { // (a nearly full card: smaller chunks)
+        if (chunk <= 128) {
+            fprintf(stderr, "llm_prefill: cannot allocate the activations of %d tokens up to position %d\n", chunk, pos0 + n);
+            return -1;
+        }
+        chunk = (chunk + 1) / 2;
+        if (m->pf_cap > chunk) { // what the larger chunk took goes back first
+            hipFree(m->pf_acc);
+            m->pf_acc = nullptr;
+            m->pf_cap = 0;
+        }
+    }
+    for (int i = 0; i < n; i += chunk) {
+        const int M = std::min(chunk, n - i);
         if (prefill_chunk(m, ids + i, pos0 + i, M)) return -1;
         if (hist && prefill_logits(m, pos0 + i, M)) return -1;
         if (i + M == n)

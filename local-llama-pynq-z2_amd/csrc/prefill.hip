@@ -1781,8 +1781,13 @@ hipError_t launch_p_embed(const ProwArgs &a, hipStream_t st) {
 hipError_t launch_p_norm_quant(const ProwArgs &a, bool resid, hipStream_t st) {
     if (a.dim % 4 || ((uintptr_t)a.oq & 3)) return hipErrorInvalidValue;
     // dim floats, a float per wave for the block sum, then the strict mode's squares and sequential sum's scratch
-    const int nt = row_threads(a.dim, a.M, a.strict);
-    const size_t lds = (size_t)(a.dim + 16) * 4 + (a.strict ? (size_t)a.dim * 4 + seq_sum_scratch_bytes(nt) : 0);
+    // (256 threads where more would not leave room for the widest rows that fit)
+    auto lds_of = [&](int nt) {
+        return (size_t)(a.dim + 8) * 4 + 32 + (a.strict ? (size_t)a.dim * 4 + seq_sum_scratch_bytes(nt) : 0);
+    };
+    int nt = row_threads(a.dim, a.M, a.strict);
+    if (lds_of(nt) > 65536) nt = 256;
+    const size_t lds = lds_of(nt);
     if (resid) hipLaunchKernelGGL(k_p_norm_quant<true>, dim3(a.M), dim3(nt), lds, st, a);
     else hipLaunchKernelGGL(k_p_norm_quant<false>, dim3(a.M), dim3(nt), lds, st, a);
     return hipGetLastError();
