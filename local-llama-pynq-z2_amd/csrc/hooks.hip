@@ -313,6 +313,9 @@ extern "C" int mvh_ref_expf_host(const float *x, int n, float *y) {
     return 0;
 }
 
+// The rule that picks the decode step's launches for long contexts (host only).
+extern "C" int mvh_step_long_ctx(int strict, int captured, int pos) { return step_long_ctx(strict, captured, pos); }
+
 extern "C" int mvh_gemv_shape(int rows, int n, int gs, int wbits, int sf32, int rb, int role, int ordered, int cus,
                               int *out) {
     static const int pro[6] = {PRO_NORM, PRO_ATTN, PRO_NORM, PRO_XQ, PRO_NORM, PRO_XQ};

@@ -149,3 +149,11 @@ def test_bin_layout(tmp_path):
     for nel in [vocab * dim] + [dim * dim] * L + [dim * kv] * (2 * L) + [dim * dim] * L + [dim * hid] * (3 * L):
         size += nel + nel // gs * 4
     assert size == len(b)
+
+
+@pytest.mark.parametrize("strict,captured,first", [(1, 0, 191), (1, 1, 191), (0, 0, 1023), (0, 1, None)])
+def test_captured_fast_steps_keep_the_short_context_launches(strict, captured, first):
+    """the position from which a decode step takes the launches for long contexts: a captured fast step never does"""
+    rule = pkg().lib().mvh_step_long_ctx
+    for pos in (0, 190, 191, 192, 1022, 1023, 1024, 3001, 131071):
+        assert rule(strict, captured, pos) == (first is not None and pos >= first)
