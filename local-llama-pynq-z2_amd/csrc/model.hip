@@ -101,6 +101,7 @@ struct llm_model {
     float *pf_ml = nullptr, *pf_acc = nullptr; // attention slice partials
     float *pf_sc = nullptr;                    // strict attention: score rows, pf_sc_n floats
     size_t pf_sc_n = 0;
+    size_t pf_limit = SIZE_MAX, pf_sc_limit = SIZE_MAX; // bytes that one of these / the score rows may take (tests)
     int8_t *pf_a = nullptr;
     int *pf_ids = nullptr;
     // h of the SwiGLU in the gate/up GEMM's epilogue (the down GEMM's input; pf_a is the gate/up input then),
@@ -889,29 +890,40 @@ int load_bin(llm_model *m, const char *path) {
 // shape) from 9456 to 8297; 4096 measured within 3% of 2048 for twice the activation memory (0.9 GB at the 7B shape).
 const int PREFILL_CHUNK = 2048;
 
-int prefill_alloc(llm_model *m, int M) {
-    if (M <= m->pf_cap) return 0;
-    const llm_info &I = m->info;
-    const int dim = I.dim, hid = I.hidden_dim, rows = std::max(dim + 2 * m->kv_dim, 2 * hid), wmax = std::max(dim, hid);
+template <typename T>
+int pf_malloc(T **p, size_t bytes, size_t limit) {
+    if (bytes <= limit && hipMalloc(p, bytes) == hipSuccess) return 0;
+    hipGetLastError();
+    *p = nullptr;
+    return -1;
+}
+
+void prefill_drop(llm_model *m) {
     auto drop = [](auto *&p) {
         if (p) hipFree(p);
         p = nullptr;
     };
     drop(m->pf_x), drop(m->pf_y), drop(m->pf_q), drop(m->pf_s), drop(m->pf_a), drop(m->pf_ids), drop(m->pf_ml);
-    drop(m->pf_acc), drop(m->pf_h), drop(m->pf_hs);
+    drop(m->pf_acc), drop(m->pf_h), drop(m->pf_hs), drop(m->pf_sc);
     m->pf_cap = 0;
-    // the GEMM input in token-block tiles (rounded up to 16 tokens, whole chunk pairs and scale quads)
-    if (hipMalloc(&m->pf_x, (size_t)M * dim * 4) != hipSuccess || hipMalloc(&m->pf_y, (size_t)M * rows * 4) != hipSuccess ||
-        hipMalloc(&m->pf_q, (size_t)M * dim * 4) != hipSuccess ||
-        hipMalloc(&m->pf_s, pf_scale_floats(wmax / m->gs, M) * 4) != hipSuccess ||
-        hipMalloc(&m->pf_a, pf_act_bytes(wmax, M)) != hipSuccess || hipMalloc(&m->pf_ids, (size_t)M * 4) != hipSuccess ||
-        hipMalloc(&m->pf_ml, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * 2 * 4) != hipSuccess ||
-        hipMalloc(&m->pf_acc, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * m->hs * 4) != hipSuccess ||
-        hipMalloc(&m->pf_h, pf_act_bytes(hid, M)) != hipSuccess ||
-        hipMalloc(&m->pf_hs, pf_scale_floats(hid / m->gs, M) * 4) != hipSuccess) {
-        hipGetLastError();
+    m->pf_sc_n = 0;
+}
+
+int prefill_alloc(llm_model *m, int M) {
+    if (M <= m->pf_cap) return 0;
+    const llm_info &I = m->info;
+    const int dim = I.dim, hid = I.hidden_dim, rows = std::max(dim + 2 * m->kv_dim, 2 * hid), wmax = std::max(dim, hid);
+    prefill_drop(m);
+    // the GEMM input in token-block tiles (rounded up to 32 tokens, whole chunk pairs and scale quads)
+    const size_t lim = m->pf_limit;
+    if (pf_malloc(&m->pf_x, (size_t)M * dim * 4, lim) || pf_malloc(&m->pf_y, (size_t)M * rows * 4, lim) ||
+        pf_malloc(&m->pf_q, (size_t)M * dim * 4, lim) || pf_malloc(&m->pf_s, pf_scale_floats(wmax / m->gs, M) * 4, lim) ||
+        pf_malloc(&m->pf_a, pf_act_bytes(wmax, M), lim) || pf_malloc(&m->pf_ids, (size_t)M * 4, lim) ||
+        pf_malloc(&m->pf_ml, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * 2 * 4, lim) ||
+        pf_malloc(&m->pf_acc, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * m->hs * 4, lim) ||
+        pf_malloc(&m->pf_h, pf_act_bytes(hid, M), lim) ||
+        pf_malloc(&m->pf_hs, pf_scale_floats(hid / m->gs, M) * 4, lim))
         return -1;
-    }
     m->pf_cap = M;
     return 0;
 }
@@ -923,12 +935,8 @@ int prefill_alloc_strict(llm_model *m, int M, int end) {
     const size_t need = prefill_strict_scratch_floats(M, m->info.n_heads, m->info.n_kv_heads, end);
     if (need <= m->pf_sc_n) return 0;
     if (m->pf_sc) hipFree(m->pf_sc);
-    m->pf_sc = nullptr;
     m->pf_sc_n = 0;
-    if (hipMalloc(&m->pf_sc, need * 4) != hipSuccess) {
-        hipGetLastError();
-        return -1;
-    }
+    if (pf_malloc(&m->pf_sc, need * 4, m->pf_sc_limit)) return -1;
     m->pf_sc_n = need;
     return 0;
 }
@@ -1100,18 +1108,17 @@ int prefill_logits(llm_model *m, int p0, int M) {
 // partials, and (finalize) its argmax into gen[pos0 + n - 1].  Afterwards the step state is position
 // pos0 + n - 1, as after those forward() calls.
 int prefill_all(llm_model *m, const int *ids, int n, bool sampled = false, int pos0 = 0, bool hist = false) {
+    // on a nearly full card: chunks down to 128 tokens, then the strict attention without score rows
     int chunk = std::min(n, PREFILL_CHUNK);
-    while (prefill_alloc(m, chunk) || prefill_alloc_strict(m, chunk, pos0 + n)) { // (a nearly full card: smaller chunks)
+    for (;;) {
+        const bool room = !prefill_alloc(m, chunk);
+        if (room && (!prefill_alloc_strict(m, chunk, pos0 + n) || chunk <= 128)) break;
         if (chunk <= 128) {
-            fprintf(stderr, "llm_prefill: cannot allocate the activations of %d tokens up to position %d\n", chunk, pos0 + n);
+            fprintf(stderr, "llm_prefill: cannot allocate the activations of %d tokens\n", chunk);
             return -1;
         }
         chunk = (chunk + 1) / 2;
-        if (m->pf_cap > chunk) { // what the larger chunk took goes back first
-            hipFree(m->pf_acc);
-            m->pf_acc = nullptr;
-            m->pf_cap = 0;
-        }
+        if (m->pf_cap > chunk) prefill_drop(m); // what the larger chunk took goes back first
     }
     for (int i = 0; i < n; i += chunk) {
         const int M = std::min(chunk, n - i);
@@ -1134,10 +1141,7 @@ void free_model(llm_model *m) {
     drop_graphs(m, false);
     for (void *p : m->allocs) hipFree(p);
     if (m->hist) hipFree(m->hist);
-    for (void *p : {(void *)m->pf_x, (void *)m->pf_y, (void *)m->pf_q, (void *)m->pf_s,
-                    (void *)m->pf_a, (void *)m->pf_ids, (void *)m->pf_ml, (void *)m->pf_acc, (void *)m->pf_h,
-                    (void *)m->pf_hs, (void *)m->pf_sc})
-        if (p) hipFree(p);
+    prefill_drop(m);
     if (m->st) hipStreamDestroy(m->st);
     if (m->file) munmap((void *)m->file, m->file_size);
     delete m;
@@ -1570,6 +1574,18 @@ extern "C" int llm_get_strict(const llm_model *m) { return m ? m->strict : -1; }
 extern "C" int llm_set_prefill(llm_model *m, int on) {
     if (!m) return -1;
     m->prefill_on = on != 0;
+    return 0;
+}
+
+// Test hook: the bytes that one prefill activation buffer and the strict score rows may take (0: any).  What the model
+// holds goes back, so that the next prompt allocates within the limits.
+extern "C" int mvh_prefill_limit(llm_model *m, size_t act_bytes, size_t score_bytes) {
+    if (!m) return -1;
+    hipSetDevice(m->device);
+    HIP_OR_FAIL("mvh_prefill_limit", hipStreamSynchronize(m->st));
+    prefill_drop(m);
+    m->pf_limit = act_bytes ? act_bytes : SIZE_MAX;
+    m->pf_sc_limit = score_bytes ? score_bytes : SIZE_MAX;
     return 0;
 }
 

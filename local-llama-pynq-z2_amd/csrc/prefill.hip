@@ -1816,9 +1816,9 @@ hipError_t launch_p_attention(const ProwArgs &a, hipStream_t st) {
             ((uintptr_t)a.oq & 3) || lds > 65536 || a.n_heads % a.n_kv ||
             (size_t)(a.p0 + a.M + 64) * a.kv_dim * 4 >= 0x7fffffffu)
             return hipErrorInvalidValue;
-        if (prefill_strict_rows(hs)) {
+        const bool by_rows = prefill_strict_rows(hs) && a.att_sc; // (no room for score rows: the general kernel)
+        if (by_rows) {
             const int kvm = a.n_heads / a.n_kv, rows = a.M * kvm, SP = prefill_strict_sp(a.p0 + a.M);
-            if (!a.att_sc) return hipErrorInvalidValue;
             // rows per wave: 4 from 14 rows per SIMD, 2 from 5.5, else 1 (whole strict prefills of two layers, 1024 SIMDs,
             // R = 4 / 2 / 1, us: Qwen2-0.5B shape 200 tokens, 2800 rows: 245 / 231 / 222; 512, 7168 rows: 328 / 306 / 320;
             // 1024, 14336 rows: 490 / 473 / 524; 2011: 943 / 990 / 1204; 7B shape 200, 5600 rows: 800 / 778 / 782; 512,
@@ -1838,7 +1838,7 @@ hipError_t launch_p_attention(const ProwArgs &a, hipStream_t st) {
             hipLaunchKernelGGL(k_p_attn_strict<0>, dim3(a.n_heads, a.M), dim3(256), lds, st, a);
         }
         hipError_t e = hipGetLastError();
-        if (e != hipSuccess || (prefill_strict_rows(hs) && hs % a.gs == 0)) return e;
+        if (e != hipSuccess || (by_rows && hs % a.gs == 0)) return e;
         hipLaunchKernelGGL(k_p_quant_rows, dim3(a.M), dim3(256), (size_t)a.dim * 4, st, a);
         return hipGetLastError();
     }

@@ -5,6 +5,7 @@ the reference's matmul (qwen.c:436-456, runq.c:429-458) exactly: the bar for it 
 oracle's sequential matvec, token by token.  The whole prefill is held to the model bars of
 test_gpu_model.py: logits within 1e-3 of the reference on the tiny models, the same greedy ids when the
 generation continues from it, and the per-position decode path's KV cache within fp32 reordering."""
+import ctypes as C
 import json
 import os
 
@@ -69,6 +70,12 @@ def test_prefill_gemm_bit_exact_special_scales(bits, shape):
     xq[4:8] = 127
     xs = rng.uniform(1e-3, 1e-1, size=(M, n // 32)).astype(np.float32)
     check_qwen_gemm(w, s, xq, xs, M, n, d, bits, 16, shape)
+
+
+def limit_prefill(m, act_bytes, score_bytes):
+    """the bytes that one prefill activation buffer and the strict score rows of `m` may take (0: any)"""
+    m.L.mvh_prefill_limit.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t]
+    assert m.L.mvh_prefill_limit(m.h, act_bytes, score_bytes) == 0
 
 
 @pytest.mark.parametrize("M,n,d,rb", [(1, 64, 36, 16), (33, 128, 100, 8), (64, 896, 64, 16), (95, 4864, 160, 8),
@@ -385,3 +392,28 @@ def test_logits_history_through_the_batched_prompt(tmp_path, fmt, shape, n, stri
     else:
         err = [rel_err(y, x) for x, y in zip(lg_a[:n], lg_b[:n])]
         assert max(err) < 2e-2 and np.median(err) < 1e-3, err
+
+
+@pytest.mark.parametrize("dim,chunk,rows", [(256, 350, True), (256, 175, False), (512, 128, False), (384, 700, False)])
+def test_strict_prefill_within_little_memory(tmp_path, dim, chunk, rows):
+    """a strict prompt of 700 tokens where the activations fit `chunk` tokens only, and where no score row fits (rows
+    False: the attention kernel that needs none, at 128 tokens or fewer): K/V rows and logits bitwise those of the
+    unlimited run.  Head sizes 64, 128 and 96"""
+    p = synth("qwb", str(tmp_path / "m.qwb"), "tiny", 17, f"dim={dim}", "heads=4", "kv_heads=2", "hidden=256", "layers=2",
+              "vocab=512", "head_k=256", "max_seq=720")
+    m = pkg().Model(p, 720)
+    m.set_strict(True)
+    ids = [int(m.head_ids[v]) for v in np.random.default_rng(dim).integers(0, 256, 700)]
+    ref = m.prefill(ids), kv_rows(m, 700)
+    acc = 4 * 16 * dim # the largest activation buffer: a token's attention partials
+    limit_prefill(m, acc * chunk, 0 if rows else 4)
+    got = m.prefill(ids), kv_rows(m, 700)
+    assert np.array_equal(ref[0], got[0])
+    for (ka, va), (kb, vb) in zip(ref[1], got[1]):
+        assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+    limit_prefill(m, acc * 127, 0)
+    with pytest.raises(RuntimeError):
+        m.prefill(ids[:128])
+    limit_prefill(m, 0, 0)
+    assert np.array_equal(ref[0], m.prefill(ids))
+    m.close()
