@@ -922,8 +922,10 @@ int prefill_alloc(llm_model *m, int M) {
         pf_malloc(&m->pf_ml, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * 2 * 4, lim) ||
         pf_malloc(&m->pf_acc, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * m->hs * 4, lim) ||
         pf_malloc(&m->pf_h, pf_act_bytes(hid, M), lim) ||
-        pf_malloc(&m->pf_hs, pf_scale_floats(hid / m->gs, M) * 4, lim))
+        pf_malloc(&m->pf_hs, pf_scale_floats(hid / m->gs, M) * 4, lim)) {
+        prefill_drop(m); // (the buffers that did fit)
         return -1;
+    }
     m->pf_cap = M;
     return 0;
 }
@@ -1578,15 +1580,20 @@ extern "C" int llm_set_prefill(llm_model *m, int on) {
 }
 
 // Test hook: the bytes that one prefill activation buffer and the strict score rows may take (0: any).  What the model
-// holds goes back, so that the next prompt allocates within the limits.
+// holds goes back, so that the next prompt allocates within the limits.  Returns the buffers it held, or -1.
 extern "C" int mvh_prefill_limit(llm_model *m, size_t act_bytes, size_t score_bytes) {
     if (!m) return -1;
     hipSetDevice(m->device);
     HIP_OR_FAIL("mvh_prefill_limit", hipStreamSynchronize(m->st));
+    int held = 0;
+    for (const void *p : {(void *)m->pf_x, (void *)m->pf_y, (void *)m->pf_q, (void *)m->pf_s, (void *)m->pf_a,
+                          (void *)m->pf_ids, (void *)m->pf_ml, (void *)m->pf_acc, (void *)m->pf_h, (void *)m->pf_hs,
+                          (void *)m->pf_sc})
+        held += p != nullptr;
     prefill_drop(m);
     m->pf_limit = act_bytes ? act_bytes : SIZE_MAX;
     m->pf_sc_limit = score_bytes ? score_bytes : SIZE_MAX;
-    return 0;
+    return held;
 }
 
 extern "C" void llm_close(llm_model *m) {
