@@ -108,8 +108,10 @@ int llm_profile_graph(llm_model *m, int steps, int rounds, llm_kernel_stat *stat
  * position n-1.  Returns 0 or -1. */
 int llm_prefill(llm_model *m, const int *ids, int n, float *logits);
 /* Whether llm_generate runs the prompt through llm_prefill (on by default) or one decode step per prompt
- * position.  A generation that keeps every position's
- * logits takes the prompt through it too, the head as one GEMM (where its row count is a multiple of 4). */
+ * position.  A generation that keeps every position's logits takes the prompt through it too, with the head as
+ * one GEMM, where the head's row count is a multiple of 4 and the activations fit; otherwise position by position.
+ * In the fast mode the two add in different orders, and so do the rows of one history: the prompt's rows come from
+ * the GEMM, its last row and the generated ones from the decode step's head. */
 int llm_set_prefill(llm_model *m, int on);
 
 /* Reference-order ("strict") mode on or off; no counterpart in the reference, whose CPU loops are this order

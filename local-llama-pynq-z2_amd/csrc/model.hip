@@ -1070,8 +1070,8 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
     return 0;
 }
 
-// Whether the head runs as a prefill GEMM (launch_pgemm's limits); otherwise a generation that keeps every position's
-// logits runs its prompt position by position.
+// Whether the head runs as a prefill GEMM (launch_pgemm's limits); otherwise, and where the prefill has no room or does
+// not take the model's shape, a generation that keeps every position's logits runs its prompt position by position.
 bool head_gemm_ok(const llm_model *m) { return m->head.rows % 4 == 0 && m->head.bytes < ((size_t)1 << 31); }
 
 // The logits of a chunk's M positions (their residual streams in pf_x) into hist rows p0 .. p0 + M - 1: the final norm
@@ -1116,7 +1116,7 @@ int prefill_all(llm_model *m, const int *ids, int n, bool sampled = false, int p
         const bool room = !prefill_alloc(m, chunk);
         if (room && (!prefill_alloc_strict(m, chunk, pos0 + n) || chunk <= 128)) break;
         if (chunk <= 128) {
-            fprintf(stderr, "llm_prefill: cannot allocate the activations of %d tokens\n", chunk);
+            if (!hist) fprintf(stderr, "llm_prefill: cannot allocate the activations of %d tokens\n", chunk);
             return -1;
         }
         chunk = (chunk + 1) / 2;
@@ -1263,7 +1263,7 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
     const int end_prompt = pos0 + n_prompt; // positions below take their token from the prompt
     // positions: the prompt, then one per generated token, within the context
     const int last_pos = std::min(end_prompt - 1 + max_new - 1, m->ctx - 1);
-    const bool batched = m->prefill_on && n_prompt > 1 && (!hist || head_gemm_ok(m));
+    bool batched = m->prefill_on && n_prompt > 1 && (!hist || head_gemm_ok(m));
     // the captured steps this run launches (both kinds where it crosses their border), before any work is queued
     const int first_step = batched ? end_prompt : pos0;
     if (first_step <= last_pos && (!step_graph(m, hist, smp, first_step) || !step_graph(m, hist, smp, last_pos)))
@@ -1277,9 +1277,16 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
     HIP_OR_FAIL("llm_generate", hipMemcpy(m->prompt + pos0, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice));
     if (set_ctrl(m, pos0 - 1, 0, end_prompt, 1)) return -1;
     const double t0 = now_ms();
+    // the prompt in one batched pass; the first decode step then finishes its last position's argmax
+    if (batched && prefill_all(m, prompt, n_prompt, smp, pos0, hist)) {
+        if (!hist) return -1;
+        // (the steps need none of the prefill's memory and write every cache row and logits row of the prompt again)
+        HIP_OR_FAIL("llm_generate", hipStreamSynchronize(m->st));
+        if (!step_graph(m, hist, smp, pos0) || !step_graph(m, hist, smp, last_pos)) return -1;
+        if (set_ctrl(m, pos0 - 1, 0, end_prompt, 1)) return -1;
+        batched = false;
+    }
     if (batched) {
-        // the prompt in one batched pass; the first decode step then finishes its last position's argmax
-        if (prefill_all(m, prompt, n_prompt, smp, pos0, hist)) return -1;
         if (set_ctrl(m, end_prompt - 1, prompt[n_prompt - 1], end_prompt, 1)) return -1;
     } else {
         for (int p = 0; p < n_prompt; p++)

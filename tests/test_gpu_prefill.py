@@ -420,3 +420,28 @@ def test_strict_prefill_within_little_memory(tmp_path, dim, chunk, rows):
     assert limit_prefill(m, 0, 0) == 0 # nothing is kept of a set that did not fit
     assert np.array_equal(ref[0], m.prefill(ids))
     m.close()
+
+
+@pytest.mark.parametrize("strict,temp", [(False, 0.0), (True, 0.8)])
+def test_logits_history_without_room_for_the_prefill(tmp_path, strict, temp):
+    """llm_generate with every position's logits where the prefill's activations do not fit: ids, logits, the sampler's
+    draws and the cache bitwise those of the position-by-position run, which needs none of them"""
+    p = synth("qwb", str(tmp_path / "h.qwb"), "tiny", 19, "dim=256", "heads=4", "kv_heads=2", "hidden=256", "layers=2",
+              "vocab=512", "head_k=256", "max_seq=300")
+    runs = []
+    for room in (False, True):
+        m = pkg().Model(p, 300)
+        ids = [int(m.head_ids[v]) for v in np.random.default_rng(4).integers(2, 256, 210)]
+        m.set_strict(strict)
+        if temp:
+            m.set_sampler(temp, 0.9, 5)
+        m.set_prefill(not room)
+        if not room:
+            limit_prefill(m, 4 * 16 * 256 * 100, 0)
+        r = m.generate(ids, 12, logits=True)
+        runs.append((r["ids"], r["logits"], kv_rows(m, 210)))
+        m.close()
+    (ids_a, lg_a, kv_a), (ids_b, lg_b, kv_b) = runs
+    assert np.array_equal(ids_a, ids_b) and np.array_equal(lg_a, lg_b)
+    for (ka, va), (kb, vb) in zip(kv_a, kv_b):
+        assert np.array_equal(ka, kb) and np.array_equal(va, vb)
