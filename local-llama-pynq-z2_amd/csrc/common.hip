@@ -1,5 +1,4 @@
 // Launch-shape choice for the GEMV kernels and the bounded stream wait (internal).
-#include <time.h>
 
 #include <algorithm>
 
@@ -125,23 +124,3 @@ GemvShape gemv_pick_shape(const TiledMat &T, int pro, int epi, int ordered, int 
 
 // Long rows with few of them (a down projection) take 8-row blocks, so that the grid still covers the chip.
 int gemv_row_block(int d, int n) { return n >= 4096 && d <= 8192 ? 8 : 16; }
-
-int stream_wait(hipStream_t st, long timeout_ms, const char *who) {
-    struct timespec t0, t;
-    clock_gettime(CLOCK_MONOTONIC, &t0);
-    for (unsigned i = 0;; i++) {
-        hipError_t e = hipStreamQuery(st);
-        if (e == hipSuccess) return 0;
-        if (e != hipErrorNotReady) {
-            fprintf(stderr, "%s: %s\n", who, hipGetErrorString(e));
-            return -1;
-        }
-        clock_gettime(CLOCK_MONOTONIC, &t);
-        const long ms = (t.tv_sec - t0.tv_sec) * 1000L + (t.tv_nsec - t0.tv_nsec) / 1000000L;
-        if (ms >= timeout_ms) return 1;
-        if (i > 64) {
-            struct timespec sl = {0, 20000};
-            nanosleep(&sl, nullptr);
-        }
-    }
-}

@@ -6,7 +6,6 @@
 #include <algorithm>
 #include <map>
 #include <string.h>
-#include <time.h>
 #include <tuple>
 #include <vector>
 
@@ -129,20 +128,6 @@ const Weight *weight(const char *who, uint64_t w, uint64_t ws, int n, int d, int
     return &S.weights.emplace(key, x).first->second;
 }
 
-// Whether the call finishes within a millisecond (the stream's own queries, which cost about 15 us each, and sleeps
-// are for the calls that do not).
-bool spin_done() {
-    struct timespec t0, t;
-    clock_gettime(CLOCK_MONOTONIC, &t0);
-    for (;;) {
-        for (int i = 0; i < (S.timeout_ms < 1 ? 1 : 256); i++)
-            if (__atomic_load_n(S.done, __ATOMIC_ACQUIRE) == S.seq) return true;
-        if (S.timeout_ms < 1) return false;
-        clock_gettime(CLOCK_MONOTONIC, &t);
-        if ((t.tv_sec - t0.tv_sec) * 1000000000L + (t.tv_nsec - t0.tv_nsec) > 1000000L) return false;
-    }
-}
-
 int run(const char *who, const Weight *W, uint64_t xq, uint64_t xs, uint64_t out, int n, int d, int gs) {
     const Buf *bx = find(xq, (size_t)n), *bxs = find(xs, (size_t)(n / gs) * 4), *bo = find(out, (size_t)d * 4);
     if (!bx || !bxs || !bo) {
@@ -190,8 +175,7 @@ int run(const char *who, const Weight *W, uint64_t xq, uint64_t xs, uint64_t out
     S.seq++;
     hipLaunchKernelGGL(k_done, dim3(1), dim3(1), 0, S.st, S.done_dev, S.seq);
     HIP_OR_FAIL(who, hipGetLastError());
-    if (spin_done()) return 0;
-    int r = S.timeout_ms < 1 ? 1 : stream_wait(S.st, S.timeout_ms, who); // (a limit of 0: one look)
+    int r = call_wait(S.done, S.seq, [] { return hipStreamQuery(S.st); }, S.timeout_ms, who);
     if (r == 1) {
         fprintf(stderr, "%s: kernel did not finish in %ld ms (n=%d d=%d)\n", who, S.timeout_ms, n, d);
         return -1;

@@ -313,6 +313,17 @@ extern "C" int mvh_ref_expf_host(const float *x, int n, float *y) {
     return 0;
 }
 
+// The drop-in call's wait on a call that never ends (host only): 1, and the microseconds it took.
+extern "C" int mvh_call_wait(long timeout_ms, double *us) {
+    static const uint32_t never = 0;
+    struct timespec t0, t1;
+    clock_gettime(CLOCK_MONOTONIC, &t0);
+    const int r = call_wait(&never, 1, [] { return hipErrorNotReady; }, timeout_ms, "mvh_call_wait");
+    clock_gettime(CLOCK_MONOTONIC, &t1);
+    *us = (t1.tv_sec - t0.tv_sec) * 1e6 + (t1.tv_nsec - t0.tv_nsec) / 1e3;
+    return r;
+}
+
 // The rule that picks the decode step's launches for long contexts (host only).
 extern "C" int mvh_step_long_ctx(int strict, int captured, int pos) { return step_long_ctx(strict, captured, pos); }
 

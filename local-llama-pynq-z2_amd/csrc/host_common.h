@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>
+#include <time.h>
 
 #include "kernels.h"
 
@@ -53,6 +54,37 @@ static inline int hip_cu_count(int dev) {
 // Row-block size for a plain matrix of d rows x n inputs (fused QKV and gate/up keep 16 for their pairing).
 int gemv_row_block(int d, int n);
 
-// Wait for the stream with a time limit (the reference's 5 s ap_done poll, matvec_fpga.cpp:34, 156-170).
-// Returns 0, 1 on time-out, -1 on a HIP error (message printed).
-int stream_wait(hipStream_t st, long timeout_ms, const char *who);
+// Wait for a call whose last launch stores seq in *done (pinned host memory), with a time limit from now on (the
+// reference's 5 s ap_done poll, matvec_fpga.cpp:34, 156-170; a limit of 0: one look).  For a millisecond the word alone is
+// looked at: a query of the stream costs about 15 us and a sleep more, and most calls end within 25.  Then `query` is
+// asked (hipSuccess, hipErrorNotReady or an error), after 64 times with sleeps between.  Returns 0, 1 on time-out, -1 on a
+// HIP error (message printed).
+template <typename Q>
+int call_wait(const uint32_t *done, uint32_t seq, Q &&query, long timeout_ms, const char *who) {
+    auto finished = [&] { return __atomic_load_n(done, __ATOMIC_ACQUIRE) == seq; };
+    if (timeout_ms < 1) return finished() ? 0 : 1;
+    struct timespec t0;
+    clock_gettime(CLOCK_MONOTONIC, &t0);
+    auto elapsed_us = [&] {
+        struct timespec t;
+        clock_gettime(CLOCK_MONOTONIC, &t);
+        return (t.tv_sec - t0.tv_sec) * 1000000L + (t.tv_nsec - t0.tv_nsec) / 1000;
+    };
+    do {
+        for (int i = 0; i < 256; i++)
+            if (finished()) return 0;
+    } while (elapsed_us() < 1000);
+    for (unsigned i = 0;; i++) {
+        const hipError_t e = query();
+        if (e == hipSuccess) return 0;
+        if (e != hipErrorNotReady) {
+            fprintf(stderr, "%s: %s\n", who, hipGetErrorString(e));
+            return -1;
+        }
+        if (elapsed_us() / 1000 >= timeout_ms) return 1;
+        if (i > 64) {
+            struct timespec sl = {0, 20000};
+            nanosleep(&sl, nullptr);
+        }
+    }
+}

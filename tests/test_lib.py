@@ -157,3 +157,15 @@ def test_captured_fast_steps_keep_the_short_context_launches(strict, captured, f
     rule = pkg().lib().mvh_step_long_ctx
     for pos in (0, 190, 191, 192, 1022, 1023, 1024, 3001, 131071):
         assert rule(strict, captured, pos) == (first is not None and pos >= first)
+
+
+@pytest.mark.parametrize("limit", [0, 1, 3])
+def test_the_drop_in_time_limit_counts_from_the_call(limit):
+    """the wait of a call that never ends takes its limit (0: one look), not the limit and the millisecond that it
+    spends on the completion word alone; the shortest of 20 (a busy machine only adds)"""
+    import ctypes as C
+    us, best = C.c_double(0), float("inf")
+    for _ in range(20):
+        assert pkg().lib().mvh_call_wait(C.c_long(limit), C.byref(us)) == 1
+        best = min(best, us.value)
+    assert 1000 * limit <= best < 1000 * limit + 900
