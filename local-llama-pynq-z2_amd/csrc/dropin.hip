@@ -136,8 +136,11 @@ int run(const char *who, const Weight *W, uint64_t xq, uint64_t xs, uint64_t out
     }
     // The GEMV reads the call's activations from pinned host memory and stores its outputs there: no copy command before
     // or after it (a call was bound by its two copies in, one out and the wait: 57-89 us at 288 x 288 to 65536 x 896; a
-    // launch that brings the activations to HBM first 14-26 us, this 12-23).  Ranges at addresses that the kernel cannot read or write as aligned vectors go through aligned
-    // device buffers (the reference's driver takes any address for fpga_matvec).
+    // launch that brings the activations to HBM first 14-26 us, this 12-23).  Every block reads the activations, which
+    // stays below the copies at long rows too (copies / this, us: 3584 x 18944 in 4 bits 38-50 / 19, .bin groups of 32
+    // 180 / 128, of 64 180 / 106; 128 x 18944 36 / 19, 180 / 98, 108 / 76).  Ranges at addresses that the kernel cannot
+    // read or write as aligned vectors go through aligned device buffers (the reference's driver takes any address for
+    // fpga_matvec).
     int8_t *xdev = (int8_t *)(bx->hdev + (xq - (uint64_t)bx->dev));
     float *sdev = (float *)(bxs->hdev + (xs - (uint64_t)bxs->dev)), *odev = (float *)(bo->hdev + (out - (uint64_t)bo->dev));
     if (xq & 15) {
