@@ -72,15 +72,6 @@ def test_prefill_gemm_bit_exact_special_scales(bits, shape):
     check_qwen_gemm(w, s, xq, xs, M, n, d, bits, 16, shape)
 
 
-def limit_prefill(m, act_bytes, score_bytes):
-    """the bytes that one prefill activation buffer and the strict score rows of `m` may take (0: any); returns how many
-    of them it held"""
-    m.L.mvh_prefill_limit.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t]
-    held = m.L.mvh_prefill_limit(m.h, act_bytes, score_bytes)
-    assert held >= 0
-    return held
-
-
 @pytest.mark.parametrize("M,n,d,rb", [(1, 64, 36, 16), (33, 128, 100, 8), (64, 896, 64, 16), (95, 4864, 160, 8),
                                       (31, 192, 32, 32), (600, 256, 1152, 16)])
 def test_prefill_gemm32_exact_and_fast(M, n, d, rb):
@@ -142,13 +133,23 @@ def test_generate_through_prefill_matches_reference_ids(name, ctx):
     assert list(r["ids"]) == meta["ids"]
 
 
+def limit_prefill(m, act_bytes, score_bytes):
+    """the bytes that one prefill activation buffer and the strict score rows of `m` may take (0: any); returns how many
+    of them it held"""
+    m.L.mvh_prefill_limit.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t]
+    held = m.L.mvh_prefill_limit(m.h, act_bytes, score_bytes)
+    assert held >= 0
+    return held
+
+
 def kv_rows(m, n_pos):
     kv = m.info.dim // m.info.n_heads * m.info.n_kv_heads
     return [(m.read_state(1, l)[:n_pos * kv], m.read_state(2, l)[:n_pos * kv]) for l in range(m.info.n_layers)]
 
 
 def test_prefill_equals_the_per_position_path_across_chunks(tmp_path):
-    """a 600-token prompt (two prefill chunks: 512 + 88) against 600 decode steps: logits of the last position,
+    """a 600-token prompt in two prefill chunks of 300 (all that its memory allows) against 600 decode steps: logits of the
+    last position,
     and every layer's K/V rows position by position.  Layer 0's rows agree to fp32 rounding; later layers may
     differ at the few positions where an activation re-quantized between the two paths' different fp32 sum
     orders crossed an int8 boundary (the flip-limited bar of test_gpu_model.py)"""
@@ -156,6 +157,7 @@ def test_prefill_equals_the_per_position_path_across_chunks(tmp_path):
     a, b = pkg().Model(p, 700), pkg().Model(p, 700)
     hid = a.head_ids
     ids = [int(hid[v]) for v in np.random.default_rng(8).integers(0, len(hid), 600)]
+    limit_prefill(a, 4 * 16 * a.info.dim * 300, 0) # (16 partials a head: the largest buffer)
     lg_pf = a.prefill(ids)
     for pos, t in enumerate(ids):
         lg_fw = b.forward(t, pos)
@@ -445,3 +447,30 @@ def test_logits_history_without_room_for_the_prefill(tmp_path, strict, temp):
     assert np.array_equal(ids_a, ids_b) and np.array_equal(lg_a, lg_b)
     for (ka, va), (kb, vb) in zip(kv_a, kv_b):
         assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+
+
+@pytest.mark.parametrize("R", [4, 2])
+@pytest.mark.parametrize("dim,heads,kv", [(896, 14, 2), (1024, 8, 2), (768, 16, 16), (512, 16, 4), (256, 16, 2)])
+def test_strict_prefill_attention_rows_per_wave(tmp_path, dim, heads, kv, R):
+    """strict prefill of as many tokens as give each wave of the attention four rows (from 14 (token, head) rows per SIMD)
+    or two (from 5.5), behind 37 earlier positions, the last tile of rows partial: K/V rows of three layers and the last
+    logits bitwise those of the decode steps, whose attention is another kernel (held to the oracle in
+    test_gpu_strict.py).  Head sizes 64, 128, 48, 32 and 16"""
+    need = (14336 if R == 4 else 5632) // heads
+    M = need + next(k for k in range(1, 17) if (need + k) * (heads // kv) % 16)
+    end = 37 + M
+    p = synth("qwb", str(tmp_path / "r.qwb"), "tiny", 23, f"dim={dim}", f"heads={heads}", f"kv_heads={kv}", "hidden=256",
+              "layers=3", "vocab=512", "head_k=256", f"max_seq={end}")
+    a, b = pkg().Model(p, end), pkg().Model(p, end)
+    ids = [int(a.head_ids[v]) for v in np.random.default_rng(M).integers(0, 256, end)]
+    for m in (a, b):
+        m.set_strict(True)
+    a.prefill(ids[:37])
+    a.continue_at(37, ids[37:], 1)
+    for pos, t in enumerate(ids):
+        lg = b.forward(t, pos)
+    for (ka, va), (kb, vb) in zip(kv_rows(a, end), kv_rows(b, end)):
+        assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+    assert np.array_equal(a.forward(ids[-1], end - 1), lg)
+    a.close()
+    b.close()
