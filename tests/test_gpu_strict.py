@@ -302,3 +302,59 @@ def test_strict_long_context_decode_equals_the_oracle(tmp_path, fmt, shape):
     m.set_prefill(False)
     assert np.array_equal(m.generate(ids, 1, logits=True)["logits"], ref)
     m.close()
+
+
+def overflowing_bin(path, dim, heads, kv, hidden=256, vocab=512):
+    """a two-layer .bin whose first layer overflows float32 at some positions and not at others: the scores of kv head
+    0's query heads (deviation 1.2e38) and the values of the last kv head (5e36, divided by the activation scales in the
+    group terms)"""
+    synth("bin", path, "tiny", 29, f"dim={dim}", f"heads={heads}", f"kv_heads={kv}", f"hidden={hidden}", "layers=2",
+          f"vocab={vocab}", "max_seq=300")
+    hs, rep = dim // heads, heads // kv
+    m = pkg().Model(path, 300)
+    m.set_strict(True)
+    m.prefill(list(range(2, 102)))
+    k, v = (m.read_state(w, 0)[:100 * kv * hs].reshape(100, kv * hs) for w in (1, 2))
+    sk, sv = float(k[:, :hs].std()), float(v[:, -hs:].std())
+    m.close()
+    f = np.fromfile(path, np.uint8)
+    wq = 256 + (2 * 2 + 1) * dim * 4 + vocab * dim // 32 * 36 # past the norms and the token table
+    wk = wq + 2 * dim * dim // 32 * 36
+    wv = wk + 2 * kv * hs * dim // 32 * 36
+    for off, d, rows, factor in ((wq, dim, slice(0, rep * hs), 1.2e4 / (sk * np.sqrt(hs))), # (queries as large as keys)
+                                 (wk, kv * hs, slice(0, hs), 1e34 / sk), (wv, kv * hs, slice(-hs, None), 5e36 / sv)):
+        at = off + d * dim # layer 0's scales
+        sc = f[at:at + d * dim // 32 * 4].view(np.float32).reshape(d, dim // 32)
+        sc[rows] = (sc[rows].astype(np.float64) * factor).astype(np.float32)
+    f.tofile(path)
+
+
+@pytest.mark.parametrize("dim,heads,kv", [(256, 4, 2), (512, 4, 4), (192, 4, 2), (256, 8, 2)])
+def test_strict_attention_with_infinities_and_nan(tmp_path, dim, heads, kv):
+    """keys and values near the largest float32: scores of +-inf and NaN, probabilities of 0 beside values of inf.  The
+    batched prefill (row kernel), the decode steps (one kernel per head below 192 positions, scores and values apart
+    from there) and the oracle agree bit for bit at every position (NaN where the others have NaN): what a later
+    position holds reaches no earlier one.  Head sizes 64, 128, 48 and 32"""
+    p = str(tmp_path / "inf.bin")
+    overflowing_bin(p, dim, heads, kv)
+    n = 260
+    ids = [int(t) for t in np.random.default_rng(dim).integers(2, 512, n)]
+    om = OracleModel(p, 300)
+    ref = np.stack([om.forward(t, pos) for pos, t in enumerate(ids)])
+    om.close()
+    a, b = pkg().Model(p, 300), pkg().Model(p, 300)
+    for m in (a, b):
+        m.set_strict(True)
+    got = a.generate(ids, 1, logits=True)["logits"]
+    for pos, t in enumerate(ids):
+        lg = b.forward(t, pos)
+        assert np.array_equal(lg, ref[pos], equal_nan=True), pos
+        assert np.array_equal(got[pos], ref[pos], equal_nan=True), pos
+    w = kv * dim // heads
+    states = [(m.read_state(i, l)[:n * w]) for l in (0, 1) for i in (1, 2) for m in (a, b)]
+    for x, y in zip(states[0::2], states[1::2]):
+        assert np.array_equal(x, y, equal_nan=True)
+    bad = ~np.isfinite(a.read_state(2, 0)[:n * w])
+    assert 0 < bad.mean() < 0.3, bad.mean() # infinities at some positions
+    a.close()
+    b.close()
