@@ -324,6 +324,9 @@ extern "C" int mvh_call_wait(long timeout_ms, double *us) {
     return r;
 }
 
+// The position slices of a decode step's attention (host only).
+extern "C" void mvh_att_slices(int pos, int splits, int *S, int *chunk) { att_slices(pos, splits, S, chunk); }
+
 // The rule that picks the decode step's launches for long contexts (host only).
 extern "C" int mvh_step_long_ctx(int strict, int captured, int pos) { return step_long_ctx(strict, captured, pos); }
 

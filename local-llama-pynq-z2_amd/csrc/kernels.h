@@ -19,14 +19,17 @@ struct StepCtrl {
 // Attention positions are processed in sub-chunks of this many rows (LDS staging of K and V).
 #define ATT_SUB 32
 
-// Position slices of one attention step: P = pos + 1 positions in S = min(splits, ceil(P / ATT_SUB)) slices
-// of `chunk` positions (the attention kernel and the o-projection's merge use the same split).
-__device__ __forceinline__ void att_slices(int pos, int splits, int *S, int *chunk) {
+// Position slices of one attention step: P = pos + 1 positions in S <= min(splits, ceil(P / ATT_SUB)) slices of `chunk`
+// positions, the last one shorter, none empty (the attention kernel and the o-projection's merge use the same split).
+// An empty slice would not be harmless: k_attention_short's buffer over T <= 0 positions would take a negative, that is
+// a huge, size, and its loads that are meant to fall outside would read 1 GiB past the cache.  From 2049 positions (64
+// slices) ceil(P / chunk) is below the slice count at one position in four.
+__host__ __device__ inline void att_slices(int pos, int splits, int *S, int *chunk) {
     const int P = pos + 1;
     int s = (P + ATT_SUB - 1) / ATT_SUB;
     if (s > splits) s = splits;
-    *S = s;
     *chunk = (P + s - 1) / s;
+    *S = (P + *chunk - 1) / *chunk;
 }
 
 

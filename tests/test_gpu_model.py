@@ -390,3 +390,23 @@ def test_fast_generation_across_1024_positions(tmp_path):
         if pos >= 1010:
             assert rel_err(m.forward(ids[k - 1], pos), lg[pos]) < 1e-3, pos
     m.close()
+
+
+@pytest.mark.parametrize("shape", [("dim=512", "heads=4", "kv_heads=2"), ("dim=384", "heads=8", "kv_heads=1")])
+def test_fast_decode_at_positions_whose_last_slice_was_empty(tmp_path, shape):
+    """fast decode steps at positions around 2049, 2201 and 3024 of a context of 4096, where 64 equal slices would leave
+    the last ones without a position: the oracle's logits, at the bars of the test across 1024 positions"""
+    p = synth("qwb", str(tmp_path / "s.qwb"), "tiny", 14, *shape, "hidden=256", "layers=1", "vocab=512", "head_k=256",
+              "max_seq=4096")
+    m, om = pkg().Model(p, 4096), OracleModel(p, 4096)
+    ids = [int(om.head_ids[v]) for v in np.random.default_rng(8).integers(2, om.n, 3027)]
+    m.prefill(ids)
+    at = {*range(2046, 2054), *range(2198, 2208), *range(3006, 3012), *range(3021, 3027)}
+    err = []
+    for pos, t in enumerate(ids):
+        ref = om.forward(t, pos)
+        if pos in at:
+            err.append(rel_err(m.forward(t, pos), ref))
+    assert max(err) < 2e-2 and np.median(err) < 1e-4, err
+    m.close()
+    om.close()

@@ -169,3 +169,16 @@ def test_the_drop_in_time_limit_counts_from_the_call(limit):
         assert pkg().lib().mvh_call_wait(C.c_long(limit), C.byref(us)) == 1
         best = min(best, us.value)
     assert 1000 * limit <= best < 1000 * limit + 900
+
+
+def test_attention_slices_cover_the_positions_and_none_is_empty():
+    """every position from 0 to 8199, and every 97th to 131071, in at most `splits` slices: the last slice holds at least
+    one position (2201 positions in 64 slices of 35 would leave the last one empty) and all of them hold every position"""
+    import ctypes as C
+    S, chunk = C.c_int(0), C.c_int(0)
+    f = pkg().lib().mvh_att_slices
+    for splits in (1, 2, 7, 35, 63, 64):
+        for pos in [*range(8200), *range(8200, 131072, 97)]:
+            f(pos, splits, C.byref(S), C.byref(chunk))
+            assert 1 <= S.value <= min(splits, pos // 32 + 1), pos
+            assert (S.value - 1) * chunk.value < pos + 1 <= S.value * chunk.value, pos
