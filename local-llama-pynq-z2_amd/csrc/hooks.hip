@@ -327,9 +327,6 @@ extern "C" int mvh_call_wait(long timeout_ms, double *us) {
 // The position slices of a decode step's attention (host only).
 extern "C" void mvh_att_slices(int pos, int splits, int *S, int *chunk) { att_slices(pos, splits, S, chunk); }
 
-// The rule that picks the decode step's launches for long contexts (host only).
-extern "C" int mvh_step_long_ctx(int strict, int captured, int pos) { return step_long_ctx(strict, captured, pos); }
-
 extern "C" int mvh_gemv_shape(int rows, int n, int gs, int wbits, int sf32, int rb, int role, int ordered, int cus,
                               int *out) {
     static const int pro[6] = {PRO_NORM, PRO_ATTN, PRO_NORM, PRO_XQ, PRO_NORM, PRO_XQ};

@@ -92,18 +92,6 @@ struct AttnArgs {
     float *one;             // fast mode, long contexts: the merged output [n_heads][hs], then (0, 1) per head
 };
 
-// Whether the decode step at position pos takes the launches for long contexts (AttnArgs::long_ctx; both kinds are right
-// at any position).  Strict, from 192 positions (a layer's step, one kernel per head / scores and values apart, us: 7B
-// shape 160 positions 73.1 / 73.0, 256 78.0 / 75.5, 3000 170 / 91; 0.5B shape 160 36.8 / 38.0, 256 39.9 / 39.0, 3000
-// 98 / 52; llama2.c 768 160 34.1 / 34.2, 256 37.1 / 35.1; 288 96 30.8 / 31.3, 160 32.4 / 31.7).  Fast, from 1024 (slices
-// merged in the o projection / merged before it: 7B shape 700 positions 58.0 / 58.0, 1200 62.1 / 59.2, 3000 66.9 / 61.0;
-// 0.5B shape 700 30.8 / 31.7, 1200 34.9 / 31.9, 3000 38.3 / 32.4; llama2.c 768 1000 32.1 / 32.2), and only outside a
-// graph: a captured fast step of 24 layers with the separate merge, at position 3001, ended in an illegal memory access
-// whose cause was not found, so captured fast steps merge in the o projection at every position.
-static inline bool step_long_ctx(bool strict, bool captured, int pos) {
-    return strict ? pos + 1 >= 192 : !captured && pos + 1 >= 1024;
-}
-
 struct EmbedArgs {
     const int8_t *emb_q;    // [vocab][dim]
     const void *emb_s;      // [vocab][dim/gs] fp16 or fp32

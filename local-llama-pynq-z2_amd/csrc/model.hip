@@ -86,7 +86,7 @@ struct llm_model {
     int part_cap = 0; // argmax partials allocated (the larger head grid of the two modes)
     StepCtrl *ctrl = nullptr;
     int *prompt = nullptr, *tokens = nullptr, *gen = nullptr;
-    // captured steps: [0 decode, 1 keeping every position's logits][sampled][0 short, 1 long contexts (strict)]
+    // captured steps: [0 decode, 1 keeping every position's logits][sampled][0 short, 1 long contexts] (step_graph)
     hipGraphExec_t g_step[2][2][2] = {};
     // on-device sampler (temperature > 0): settings and RNG on the device, scratch, the sampling step graphs
     bool sampling = false;
@@ -221,13 +221,21 @@ hipError_t launch_sampler(llm_model *m) {
     return launch_sample(a, m->st);
 }
 
+// Whether the step at `pos` takes the launches for long contexts (both kinds are right at any position).  Strict, from
+// 192 positions (a layer's step, one kernel per head / scores and values apart, us: 7B shape 160 positions 73.1 / 73.0,
+// 256 78.0 / 75.5, 3000 170 / 91; 0.5B shape 160 36.8 / 38.0, 256 39.9 / 39.0, 3000 98 / 52; llama2.c 768 160 34.1 /
+// 34.2, 256 37.1 / 35.1; 288 96 30.8 / 31.3, 160 32.4 / 31.7).  Fast, from 1024 (slices merged in the o projection /
+// merged before it: 7B shape 700 positions 58.0 / 58.0, 1200 62.1 / 59.2, 3000 66.9 / 61.0; 0.5B shape 700 30.8 / 31.7,
+// 1200 34.9 / 31.9, 3000 38.3 / 32.4; llama2.c 768 1000 32.1 / 32.2).
+bool long_step(const llm_model *m, int pos) { return pos + 1 >= (m->strict ? 192 : 1024); }
+
 // Enqueue one decode step on m->st.  prof != NULL records events around every launch.  Kernel kinds whose
 // bit is set in `skip` are left out (the in-graph timing of llm_profile_graph compares such steps).  With
-// `sampled`, the sampler follows the head.  lng: the launches for long contexts (step_long_ctx).
-int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finalize, bool lng, unsigned skip = 0,
+// `sampled`, the sampler follows the head.
+int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finalize, unsigned skip = 0,
                  bool sampled = false) {
     const llm_info &I = m->info;
-    const int dim = I.dim, kv = m->kv_dim;
+    const int dim = I.dim, kv = m->kv_dim, lng = long_step(m, pos_hint);
     auto mark = [&](int kind, double bytes) {
         if (!prof) return;
         if (prof->used + 2 > prof->ev.size()) {
@@ -382,7 +390,7 @@ int enqueue_step(llm_model *m, bool hist, Prof *prof, int pos_hint, bool finaliz
 int capture(llm_model *m, bool hist, hipGraphExec_t *out, int pos, unsigned skip = 0, bool sampled = false) {
     hipGraph_t g;
     HIP_OR_FAIL("llm", hipStreamBeginCapture(m->st, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_step(m, hist, nullptr, pos, false, step_long_ctx(m->strict, true, pos), skip, sampled);
+    int rc = enqueue_step(m, hist, nullptr, pos, false, skip, sampled);
     hipError_t e = hipStreamEndCapture(m->st, &g);
     if (rc || e != hipSuccess) {
         fprintf(stderr, "llm: graph capture failed: %s\n", hipGetErrorString(e));
@@ -399,7 +407,7 @@ int capture(llm_model *m, bool hist, hipGraphExec_t *out, int pos, unsigned skip
 
 // the captured step for position pos, captured at its first use; NULL (message printed) on failure
 hipGraphExec_t step_graph(llm_model *m, bool hist, bool sampled, int pos) {
-    hipGraphExec_t *g = &m->g_step[hist][sampled][step_long_ctx(m->strict, true, pos)];
+    hipGraphExec_t *g = &m->g_step[hist][sampled][long_step(m, pos)];
     if (!*g && capture(m, hist, g, pos, 0, sampled)) return nullptr;
     return *g;
 }
@@ -1220,7 +1228,7 @@ extern "C" int llm_forward(llm_model *m, int token, int pos, float *logits) {
     }
     hipSetDevice(m->device);
     if (set_ctrl(m, pos, token, 0, 0)) return -1;
-    if (enqueue_step(m, false, nullptr, pos, true, step_long_ctx(m->strict, false, pos))) return -1;
+    if (enqueue_step(m, false, nullptr, pos, true)) return -1;
     if (logits)
         HIP_OR_FAIL("llm_forward", hipMemcpyAsync(logits, m->logits, (size_t)m->info.n_logits * 4,
                                                   hipMemcpyDeviceToHost, m->st));
@@ -1395,7 +1403,7 @@ extern "C" int llm_profile(llm_model *m, int steps, llm_kernel_stat *stats, int 
         pr.used = 0;
         pr.kind.clear();
         pr.bytes.clear();
-        if (enqueue_step(m, false, &pr, c.pos + 1 + s, false, step_long_ctx(m->strict, false, c.pos + 1 + s))) return -1;
+        if (enqueue_step(m, false, &pr, c.pos + 1 + s, false)) return -1;
         HIP_OR_FAIL("llm_profile", hipStreamSynchronize(m->st));
         for (size_t i = 0; i < pr.kind.size(); i++) {
             float t = 0;

@@ -373,22 +373,23 @@ def test_fast_decode_across_the_long_context_switch(tmp_path, shape, ctx):
     om.close()
 
 
-def test_fast_generation_across_1024_positions(tmp_path):
-    """fast captured steps from position 1010 to 1049: every generated token is the argmax of its row of the logits
-    history, and the rows match the eager llm_forward, which merges the attention slices in a launch of its own from
-    1024 positions, within 1e-3 of their scale (the same terms in the same order)"""
+@pytest.mark.parametrize("first,ctx", [(1010, 1100), (2035, 4096), (3001, 4096)])
+def test_fast_generation_at_long_contexts(tmp_path, first, ctx):
+    """fast captured steps of a generation from position `first`: across the switch at 1024 to the launches that merge the
+    attention slices apart, across 2048 positions (64 slices) and over positions whose last slice was once empty.  Every
+    generated token is the argmax of its row of the logits history, and every row is bitwise the eager llm_forward's"""
     p = synth("qwb", str(tmp_path / "g.qwb"), "tiny", 12, "dim=512", "heads=4", "kv_heads=2", "hidden=256", "layers=2",
-              "vocab=512", "head_k=256", "max_seq=1100")
-    m = pkg().Model(p, 1100)
+              "vocab=512", "head_k=256", f"max_seq={ctx}")
+    m = pkg().Model(p, ctx)
     hid = np.asarray(m.head_ids)
-    prompt = [int(hid[v]) for v in np.random.default_rng(6).integers(2, len(hid), 1010)]
+    prompt = [int(hid[v]) for v in np.random.default_rng(6).integers(2, len(hid), first)]
     r = m.generate(prompt, 40, logits=True)
     ids, lg = [int(t) for t in r["ids"]], r["logits"]
     for k, t in enumerate(ids):
-        pos = 1009 + k
+        pos = first - 1 + k
         assert t == hid[int(np.argmax(lg[pos]))]
-        if pos >= 1010:
-            assert rel_err(m.forward(ids[k - 1], pos), lg[pos]) < 1e-3, pos
+        if k:
+            assert np.array_equal(m.forward(ids[k - 1], pos), lg[pos]), pos
     m.close()
 
 

@@ -151,14 +151,6 @@ def test_bin_layout(tmp_path):
     assert size == len(b)
 
 
-@pytest.mark.parametrize("strict,captured,first", [(1, 0, 191), (1, 1, 191), (0, 0, 1023), (0, 1, None)])
-def test_captured_fast_steps_keep_the_short_context_launches(strict, captured, first):
-    """the position from which a decode step takes the launches for long contexts: a captured fast step never does"""
-    rule = pkg().lib().mvh_step_long_ctx
-    for pos in (0, 190, 191, 192, 1022, 1023, 1024, 3001, 131071):
-        assert rule(strict, captured, pos) == (first is not None and pos >= first)
-
-
 @pytest.mark.parametrize("limit", [0, 1, 3])
 def test_the_drop_in_time_limit_counts_from_the_call(limit):
     """the wait of a call that never ends takes its limit (0: one look), not the limit and the millisecond that it
