@@ -101,7 +101,10 @@ struct llm_model {
     float *pf_ml = nullptr, *pf_acc = nullptr; // attention slice partials
     float *pf_sc = nullptr;                    // strict attention: score rows, pf_sc_n floats
     size_t pf_sc_n = 0;
-    size_t pf_limit = SIZE_MAX, pf_sc_limit = SIZE_MAX; // bytes that one of these / the score rows may take (tests)
+    size_t pf_bytes = 0;                       // what the activation matrices take
+    int pf_sets = 0;                           // times they were allocated
+    // set by tests: the bytes that one of these may take, the score rows, and all of them together
+    size_t pf_limit = SIZE_MAX, pf_sc_limit = SIZE_MAX, pf_room = SIZE_MAX;
     int8_t *pf_a = nullptr;
     int *pf_ids = nullptr;
     // h of the SwiGLU in the gate/up GEMM's epilogue (the down GEMM's input; pf_a is the gate/up input then),
@@ -900,7 +903,7 @@ const int PREFILL_CHUNK = 2048;
 
 template <typename T>
 int pf_malloc(T **p, size_t bytes, size_t limit) {
-    if (bytes <= limit && hipMalloc(p, bytes) == hipSuccess) return 0;
+    if (bytes <= limit && hipMalloc((void **)p, bytes) == hipSuccess) return 0;
     hipGetLastError();
     *p = nullptr;
     return -1;
@@ -914,40 +917,60 @@ void prefill_drop(llm_model *m) {
     drop(m->pf_x), drop(m->pf_y), drop(m->pf_q), drop(m->pf_s), drop(m->pf_a), drop(m->pf_ids), drop(m->pf_ml);
     drop(m->pf_acc), drop(m->pf_h), drop(m->pf_hs), drop(m->pf_sc);
     m->pf_cap = 0;
-    m->pf_sc_n = 0;
+    m->pf_bytes = m->pf_sc_n = 0;
 }
 
-int prefill_alloc(llm_model *m, int M) {
-    if (M <= m->pf_cap) return 0;
+// bytes that the prefill's buffers may take now, those it holds given back
+size_t pf_room(const llm_model *m) {
+    const size_t held = m->pf_bytes + m->pf_sc_n * 4;
+    size_t free_b, total;
+    if (hipMemGetInfo(&free_b, &total) != hipSuccess) {
+        hipGetLastError();
+        return m->pf_room; // (the allocations will tell)
+    }
+    return std::min(free_b + held, m->pf_room);
+}
+
+// The activation matrices of M tokens, and (score_floats) the strict attention's score rows; what is held already stays
+// where it serves.  Returns -1, and keeps what is held, where the card has no room: a nearly full card then runs every
+// prompt in the chunks that fit, without freeing and allocating for each.
+int prefill_alloc(llm_model *m, int M, size_t score_floats) {
+    if (M <= m->pf_cap && score_floats <= m->pf_sc_n) return 0;
     const llm_info &I = m->info;
     const int dim = I.dim, hid = I.hidden_dim, rows = std::max(dim + 2 * m->kv_dim, 2 * hid), wmax = std::max(dim, hid);
-    prefill_drop(m);
     // the GEMM input in token-block tiles (rounded up to 32 tokens, whole chunk pairs and scale quads)
-    const size_t lim = m->pf_limit;
-    if (pf_malloc(&m->pf_x, (size_t)M * dim * 4, lim) || pf_malloc(&m->pf_y, (size_t)M * rows * 4, lim) ||
-        pf_malloc(&m->pf_q, (size_t)M * dim * 4, lim) || pf_malloc(&m->pf_s, pf_scale_floats(wmax / m->gs, M) * 4, lim) ||
-        pf_malloc(&m->pf_a, pf_act_bytes(wmax, M), lim) || pf_malloc(&m->pf_ids, (size_t)M * 4, lim) ||
-        pf_malloc(&m->pf_ml, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * 2 * 4, lim) ||
-        pf_malloc(&m->pf_acc, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * m->hs * 4, lim) ||
-        pf_malloc(&m->pf_h, pf_act_bytes(hid, M), lim) ||
-        pf_malloc(&m->pf_hs, pf_scale_floats(hid / m->gs, M) * 4, lim)) {
-        prefill_drop(m); // (the buffers that did fit)
-        return -1;
+    const std::pair<void **, size_t> buf[] = {
+        {(void **)&m->pf_x, (size_t)M * dim * 4},
+        {(void **)&m->pf_y, (size_t)M * rows * 4},
+        {(void **)&m->pf_q, (size_t)M * dim * 4},
+        {(void **)&m->pf_s, pf_scale_floats(wmax / m->gs, M) * 4},
+        {(void **)&m->pf_a, pf_act_bytes(wmax, M)},
+        {(void **)&m->pf_ids, (size_t)M * 4},
+        {(void **)&m->pf_ml, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * 2 * 4},
+        {(void **)&m->pf_acc, (size_t)M * I.n_heads * PREFILL_ATT_SMAX * m->hs * 4},
+        {(void **)&m->pf_h, pf_act_bytes(hid, M)},
+        {(void **)&m->pf_hs, pf_scale_floats(hid / m->gs, M) * 4}};
+    size_t act = 0;
+    for (const auto &b : buf) act += b.second;
+    const size_t room = pf_room(m), score = score_floats * 4;
+    if (M > m->pf_cap || m->pf_bytes + score > room) { // the whole set again (the larger one held leaves no room)
+        if (act + score > room) return -1;
+        prefill_drop(m);
+        for (const auto &b : buf)
+            if (pf_malloc(b.first, b.second, m->pf_limit)) {
+                prefill_drop(m); // (the buffers that did fit)
+                return -1;
+            }
+        m->pf_cap = M;
+        m->pf_bytes = act;
+        m->pf_sets++;
     }
-    m->pf_cap = M;
-    return 0;
-}
-
-// the strict attention's score rows for chunks of M tokens up to position `end` (grown, never per chunk: a prompt's
-// last chunk has its largest end)
-int prefill_alloc_strict(llm_model *m, int M, int end) {
-    if (!m->strict || !prefill_strict_rows(m->hs)) return 0;
-    const size_t need = prefill_strict_scratch_floats(M, m->info.n_heads, m->info.n_kv_heads, end);
-    if (need <= m->pf_sc_n) return 0;
-    if (m->pf_sc) hipFree(m->pf_sc);
-    m->pf_sc_n = 0;
-    if (pf_malloc(&m->pf_sc, need * 4, m->pf_sc_limit)) return -1;
-    m->pf_sc_n = need;
+    if (score_floats > m->pf_sc_n) {
+        if (m->pf_sc) hipFree(m->pf_sc);
+        m->pf_sc_n = 0;
+        if (pf_malloc(&m->pf_sc, score, m->pf_sc_limit)) return -1;
+        m->pf_sc_n = score_floats;
+    }
     return 0;
 }
 
@@ -988,7 +1011,7 @@ int prefill_chunk(llm_model *m, const int *ids, int p0, int M) {
     pa.strict = m->strict;
     pa.simds = 4 * hip_cu_count(m->device);
     pa.flash_bf = m->pf_flash_bf;
-    pa.att_sc = m->pf_sc;
+    if (prefill_strict_scratch_floats(M, I.n_heads, I.n_kv_heads, p0 + M) <= m->pf_sc_n) pa.att_sc = m->pf_sc;
     pa.xb = m->pf_y; // strict attention rows: the QKV GEMM output is consumed by then
     HIP_OR_FAIL("llm_prefill", launch_p_embed(pa, m->st));
     PgemmArgs g;
@@ -1120,15 +1143,16 @@ int prefill_logits(llm_model *m, int p0, int M) {
 int prefill_all(llm_model *m, const int *ids, int n, bool sampled = false, int pos0 = 0, bool hist = false) {
     // on a nearly full card: chunks down to 128 tokens, then the strict attention without score rows
     int chunk = std::min(n, PREFILL_CHUNK);
+    const bool by_rows = m->strict && prefill_strict_rows(m->hs);
     for (;;) {
-        const bool room = !prefill_alloc(m, chunk);
-        if (room && (!prefill_alloc_strict(m, chunk, pos0 + n) || chunk <= 128)) break;
+        const size_t score =
+            by_rows ? prefill_strict_scratch_floats(chunk, m->info.n_heads, m->info.n_kv_heads, pos0 + n) : 0;
+        if (!prefill_alloc(m, chunk, score) || (chunk <= 128 && score && !prefill_alloc(m, chunk, 0))) break;
         if (chunk <= 128) {
             if (!hist) fprintf(stderr, "llm_prefill: cannot allocate the activations of %d tokens\n", chunk);
             return -1;
         }
         chunk = (chunk + 1) / 2;
-        if (m->pf_cap > chunk) prefill_drop(m); // what the larger chunk took goes back first
     }
     for (int i = 0; i < n; i += chunk) {
         const int M = std::min(chunk, n - i);
@@ -1594,9 +1618,10 @@ extern "C" int llm_set_prefill(llm_model *m, int on) {
     return 0;
 }
 
-// Test hook: the bytes that one prefill activation buffer and the strict score rows may take (0: any).  What the model
-// holds goes back, so that the next prompt allocates within the limits.  Returns the buffers it held, or -1.
-extern "C" int mvh_prefill_limit(llm_model *m, size_t act_bytes, size_t score_bytes) {
+// Test hook: the bytes that one prefill activation buffer and the strict score rows may take before their allocation
+// fails, and the room for all of them (0: any).  What the model holds goes back, so that the next prompt allocates within
+// the limits.  Returns the buffers it held, or -1.
+extern "C" int mvh_prefill_limit(llm_model *m, size_t act_bytes, size_t score_bytes, size_t room) {
     if (!m) return -1;
     hipSetDevice(m->device);
     HIP_OR_FAIL("mvh_prefill_limit", hipStreamSynchronize(m->st));
@@ -1608,7 +1633,14 @@ extern "C" int mvh_prefill_limit(llm_model *m, size_t act_bytes, size_t score_by
     prefill_drop(m);
     m->pf_limit = act_bytes ? act_bytes : SIZE_MAX;
     m->pf_sc_limit = score_bytes ? score_bytes : SIZE_MAX;
+    m->pf_room = room ? room : SIZE_MAX;
     return held;
+}
+
+// Test hook: the sets of prefill buffers allocated so far, and the bytes of the one held.
+extern "C" int mvh_prefill_sets(const llm_model *m, size_t *bytes) {
+    *bytes = m->pf_bytes;
+    return m->pf_sets;
 }
 
 extern "C" void llm_close(llm_model *m) {

@@ -133,11 +133,11 @@ def test_generate_through_prefill_matches_reference_ids(name, ctx):
     assert list(r["ids"]) == meta["ids"]
 
 
-def limit_prefill(m, act_bytes, score_bytes):
-    """the bytes that one prefill activation buffer and the strict score rows of `m` may take (0: any); returns how many
-    of them it held"""
-    m.L.mvh_prefill_limit.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t]
-    held = m.L.mvh_prefill_limit(m.h, act_bytes, score_bytes)
+def limit_prefill(m, act_bytes, score_bytes, room=0):
+    """the bytes that one prefill activation buffer and the strict score rows of `m` may take before their allocation
+    fails, and the room for all of them (0: any); returns how many of them it held"""
+    m.L.mvh_prefill_limit.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t]
+    held = m.L.mvh_prefill_limit(m.h, act_bytes, score_bytes, room)
     assert held >= 0
     return held
 
@@ -474,3 +474,36 @@ def test_strict_prefill_attention_rows_per_wave(tmp_path, dim, heads, kv, R):
     assert np.array_equal(a.forward(ids[-1], end - 1), lg)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("strict", [False, True])
+def test_prefill_on_a_nearly_full_card_keeps_its_buffers(tmp_path, strict):
+    """prompts where the set for half their tokens fits and the whole does not: one allocation for all of them, the same
+    K/V rows and logits as in chunks without that limit; a larger set once there is room"""
+    p = synth("qwb", str(tmp_path / "n.qwb"), "tiny", 37, "dim=256", "heads=4", "kv_heads=2", "hidden=256", "layers=2",
+              "vocab=512", "head_k=256", "max_seq=720")
+    m = pkg().Model(p, 720)
+    m.set_strict(strict)
+    m.L.mvh_prefill_sets.argtypes = [C.c_void_p, C.c_void_p]
+    size = C.c_size_t(0)
+    sets = lambda: m.L.mvh_prefill_sets(m.h, C.byref(size))
+    ids = [int(m.head_ids[v]) for v in np.random.default_rng(2).integers(0, 256, 700)]
+    limit_prefill(m, 4 * 16 * 256 * 350, 0) # (attention partials: the largest buffer) two chunks of 350
+    ref = m.prefill(ids), kv_rows(m, 700)
+    m.prefill(ids[:350])
+    sets()
+    score = 2 * 350 * 2 * 704 * 4 if strict else 0 # kv heads x rows of a kv head x positions
+    limit_prefill(m, 0, 0, int(1.1 * (size.value + score)))
+    before = sets()
+    for n in (700, 660, 700, 130):
+        got = m.prefill(ids[:n]), kv_rows(m, 700)
+        if n == 700:
+            assert np.array_equal(ref[0], got[0])
+            for (ka, va), (kb, vb) in zip(ref[1], got[1]):
+                assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+    assert sets() == before + 1
+    limit_prefill(m, 0, 0)
+    m.prefill(ids[:350])
+    m.prefill(ids)
+    assert sets() == before + 3
+    m.close()
