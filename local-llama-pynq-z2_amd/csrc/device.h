@@ -176,7 +176,8 @@ __device__ __forceinline__ float seq_sum(const float *p, int n) {
 // DPP row, packed little-endian, and the group's scale.  Every lane of the wave calls it (the group max is
 // max8 / max16 across lanes).
 __device__ __forceinline__ uint32_t quantize_pack(float4 x, int gs, int flavor, float *scale_out) {
-    float m = fmaxf(fmaxf(fmaxf(0.0f, fabsf(x.x)), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))); // (all NaN: 0)
+    // the reference's running maximum from 0 (a group of NaN: 0); as a chain it is two three-operand instructions
+    float m = fmaxf(fmaxf(fmaxf(fmaxf(0.0f, fabsf(x.x)), fabsf(x.y)), fabsf(x.z)), fabsf(x.w));
     m = gs == 64 ? max16(m) : max8(m);
     const float scale = quant_scale(m, flavor), inv = quant_inv(scale);
     const uint32_t b0 = (uint8_t)quant_one(x.x, scale, inv, flavor);
