@@ -101,11 +101,11 @@ int llm_profile(llm_model *m, int steps, llm_kernel_stat *stats, int max_stats);
 int llm_profile_graph(llm_model *m, int steps, int rounds, llm_kernel_stat *stats, int max_stats, double *step_ms);
 
 /* Batched prompt processing (prefill; the reference runs the prompt one forward() per position,
- * qwen.c:674-681): positions 0..n-1 pass through each layer together, in chunks of up to 512 tokens.  The
- * layer matrices become int8 MFMA GEMMs with exact int32 group sums and the reference's per-group product
- * and group order; attention is causal over the KV cache.  Fills the KV cache like n forward() calls and
- * leaves the logits of position n-1 in `logits` (n_logits floats, may be NULL); the step state is then
- * position n-1.  Returns 0 or -1. */
+ * qwen.c:674-681): positions 0..n-1 pass through each layer together, in chunks of up to 2048 tokens (smaller ones
+ * where a nearly full card has no room).  The layer matrices become int8 MFMA GEMMs with exact int32 group sums and, in
+ * the strict mode, the reference's per-group product and group order; attention is causal over the KV cache.
+ * Fills the KV cache like n forward() calls and leaves the logits of position n-1 in `logits` (n_logits floats, may
+ * be NULL); the step state is then position n-1.  Returns 0 or -1. */
 int llm_prefill(llm_model *m, const int *ids, int n, float *logits);
 /* Whether llm_generate runs the prompt through llm_prefill (on by default) or one decode step per prompt
  * position.  A generation that keeps every position's logits takes the prompt through it too, with the head as

@@ -896,9 +896,11 @@ int load_bin(llm_model *m, const char *path) {
 
 // ---- prefill (batched prompt processing)
 
-// Tokens per pass through the layers.  A chunk's kernels fill the chip only with enough tiles: 512 -> 2048 tokens took
-// four strict layers of 2011 tokens (Qwen2-0.5B shape) from 3184 to 2154 us and two fast layers of 3000 tokens (7B
-// shape) from 9456 to 8297; 4096 measured within 3% of 2048 for twice the activation memory (0.9 GB at the 7B shape).
+// Tokens per pass through the layers.  A chunk's kernels fill the chip only with enough tiles.  Chunks of 512 / 1024 /
+// 2048 tokens, us: 2011 tokens of the Qwen2-0.5B shape, four layers, strict 2846 / 2233 / 1798, fast 1835 / 1373 / 1076;
+// 3000 of the 7B shape, two fast layers, 7148 / 6347 / 6001; 4096 measured within 3% of 2048 for twice the activation
+// memory (0.9 GB at the 7B shape, and as much again for the strict score rows at 4096 positions; held until the model
+// is closed).
 const int PREFILL_CHUNK = 2048;
 
 template <typename T>
@@ -1108,8 +1110,8 @@ bool head_gemm_ok(const llm_model *m) { return m->head.rows % 4 == 0 && m->head.
 // The logits of a chunk's M positions (their residual streams in pf_x) into hist rows p0 .. p0 + M - 1: the final norm
 // per token, then the head as one GEMM.  The prompt's steps one by one read every weight once per position: 97 tokens
 // through two layers of the 0.5B shape and a 16,384-row head 6587 us, this way 649.  Strict: bitwise the steps' logits.
-// Fast: the sums are taken in another order; the logits' distance from float64, mean over 60 prompts of 24 tokens,
-// 0.00366 by steps and 0.00302 this way, over 40 of 97 tokens 0.00676 and 0.00652.
+// Fast: the sums are taken in another order; the logits' distance from float64 by steps / this way, mean over 124 prompts
+// of 24 tokens 0.00360 / 0.00350, over 124 of 97 tokens 0.00690 / 0.00688.
 int prefill_logits(llm_model *m, int p0, int M) {
     const llm_info &I = m->info;
     ProwArgs pa;
@@ -1296,7 +1298,8 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
     // positions: the prompt, then one per generated token, within the context
     const int last_pos = std::min(end_prompt - 1 + max_new - 1, m->ctx - 1);
     bool batched = m->prefill_on && n_prompt > 1 && (!hist || head_gemm_ok(m));
-    // the captured steps this run launches (both kinds where it crosses their border), before any work is queued
+    // the captured steps this run launches (both kinds where it crosses their border), before any work is queued: a
+    // capture is host work that the prompt's time would otherwise hold
     const int first_step = batched ? end_prompt : pos0;
     if (first_step <= last_pos && (!step_graph(m, hist, smp, first_step) || !step_graph(m, hist, smp, last_pos)))
         return -1;

@@ -77,8 +77,9 @@ struct PgemmArgs {
 
 // Tile shape of the prefill GEMM for d output rows and M tokens on a device of `simds` SIMDs.  The smallest
 // tile (16 x 16) needs the most instructions per output but gives the most waves; 32 x 32 tiles pay off once
-// they still give every SIMD 4 waves (measured on the 512-token Qwen2-0.5B-shape GEMMs: 32 x 32 for the
-// 9728-row gate/up, 16 x 16 for QKV, o and down).
+// they still give every SIMD 4 waves (measured on the 512-token Qwen2-0.5B-shape GEMMs, int4: 32 x 32 for the
+// 9728-row gate/up, 16 x 16 for QKV, o and down).  The model's int4 GEMMs go to k_pgemm32 where it has the waves
+// (pgemm_shape), that gate/up among them; int8 ones come here at every size.
 static inline int pgemm_pick_shape(int d, int M, int simds) {
     if (simds <= 0) simds = 1024;
     const long waves22 = (long)((d + 31) / 32) * ((M + 31) / 32);

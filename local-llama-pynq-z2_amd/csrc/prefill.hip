@@ -940,7 +940,7 @@ hipError_t launch_pgemm(int wbits, int gs, int sf32, const PgemmArgs &a, hipStre
 }
 
 // ------------------------------------------------------------------------------------------------------
-// per-token element-wise steps (one block of 256 threads per token)
+// per-token element-wise steps (one block per token, of row_threads() or 256 threads)
 
 // Threads of a per-token block: rows of up to 4 elements per thread are loaded in one round (the kernels' first NQ or
 // MP passes); longer rows run pass after pass, a round trip each, at 256 threads.  With more tokens than fill the chip
@@ -1449,7 +1449,7 @@ __global__ void __launch_bounds__(1024) k_p_attn_merge(ProwArgs a, int all) {
     if (S == 1 && !all) return;
     // fixed-trip loops with the slice count as a predicate: every load of a row is issued before the first
     // is waited for.  The value partials of this thread's first MP outputs do not depend on the weights:
-    // they are loaded first, together with the statistics (one round trip for a row of up to MP * 256 values).
+    // they are loaded first, together with the statistics (one round trip for a row of up to MP values per thread).
     constexpr int MP = 4;
     float xp[MP][PREFILL_ATT_SMAX];
 #pragma unroll
