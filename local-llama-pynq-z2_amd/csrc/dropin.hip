@@ -105,6 +105,7 @@ const Weight *weight(const char *who, uint64_t w, uint64_t ws, int n, int d, int
     x.T = tiled_describe(d, n, gs, wbits, sf32, ordered ? 64 : 16);
     if (hipMalloc(&x.tiled, x.T.bytes) != hipSuccess) {
         fprintf(stderr, "%s: cannot allocate %zu bytes of HBM for a weight matrix\n", who, x.T.bytes);
+        (void)hipGetLastError();
         return nullptr;
     }
     x.T.data = x.tiled;
@@ -243,6 +244,7 @@ extern "C" void *fpga_alloc_try(size_t bytes, uint64_t *phys) {
     if (e != hipSuccess) {
         snprintf(S.last_err, sizeof S.last_err, "%zu bytes failed after %.1f MiB already allocated: %s", bytes,
                  S.total / 1048576.0, hipGetErrorString(e));
+        (void)hipGetLastError();
         if (h) hipHostFree(h);
         return nullptr;
     }

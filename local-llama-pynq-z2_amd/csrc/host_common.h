@@ -7,12 +7,14 @@
 
 #include "kernels.h"
 
-// Print "<who>: <what>: <hip error>" to stderr and return -1 from the calling function.
+// Print "<who>: <what>: <hip error>" to stderr and return -1 from the calling function.  (An error stays the runtime's
+// last one until it is fetched, and the launchers return the last error: a reported one is taken off.)
 #define HIP_OR_FAIL(who, call)                                                                        \
     do {                                                                                             \
         hipError_t e_ = (call);                                                                      \
         if (e_ != hipSuccess) {                                                                      \
             fprintf(stderr, "%s: %s failed: %s\n", who, #call, hipGetErrorString(e_));              \
+            (void)hipGetLastError();                                                                 \
             return -1;                                                                               \
         }                                                                                            \
     } while (0)

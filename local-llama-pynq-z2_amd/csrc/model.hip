@@ -130,6 +130,7 @@ int dalloc(llm_model *m, T **p, size_t bytes) {
     void *v = nullptr;
     if (hipMalloc(&v, bytes ? bytes : 16) != hipSuccess) {
         fprintf(stderr, "llm_open: cannot allocate %zu bytes of HBM\n", bytes);
+        (void)hipGetLastError();
         return -1;
     }
     if (hipMemset(v, 0, bytes ? bytes : 16) != hipSuccess) return -1;
@@ -1291,6 +1292,8 @@ static int generate_from(llm_model *m, int pos0, const int *prompt, int n_prompt
     if (hist && !m->hist) {
         if (hipMalloc(&m->hist, (size_t)m->ctx * m->info.n_logits * 4) != hipSuccess) {
             fprintf(stderr, "llm_generate: no room for the logits history\n");
+            (void)hipGetLastError();
+            m->hist = nullptr;
             return -1;
         }
     }

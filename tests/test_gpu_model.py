@@ -19,7 +19,7 @@ import subprocess
 import numpy as np
 import pytest
 
-from helpers import GOLDEN, PKG_DIR, REF_DIR, OracleModel, pkg, rel_err, synth
+from helpers import GOLDEN, PKG_DIR, REF_DIR, OracleModel, pkg, ptr, rel_err, synth
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3
@@ -411,3 +411,16 @@ def test_fast_decode_at_positions_whose_last_slice_was_empty(tmp_path, shape):
     assert max(err) < 2e-2 and np.median(err) < 1e-4, err
     m.close()
     om.close()
+
+
+def test_generation_after_a_logits_history_that_did_not_fit(tmp_path):
+    """a context whose logits history (2,000,000 x 60,000 floats) fits no card: llm_generate with logits fails, and the next
+    generation without them runs (the failed allocation's error is not the next launch's)"""
+    import ctypes as C
+    p = synth("qwb", str(tmp_path / "o.qwb"), "tiny", 3, "dim=128", "heads=8", "kv_heads=1", "hidden=128", "layers=1",
+              "vocab=60001", "head_k=60000", "max_seq=2000000")
+    m = pkg().Model(p, 2000000)
+    ids, out, lg = np.array([5, 9, 7], np.int32), np.zeros(4, np.int32), np.zeros(4, np.float32)
+    assert m.L.llm_generate(m.h, ptr(ids), 3, 4, ptr(out), ptr(lg), None) == -1
+    assert m.L.llm_generate(m.h, ptr(ids), 3, 4, ptr(out), None, None) == 4
+    m.close()
